@@ -59,7 +59,7 @@ LDS_PEAK_GBPS = 256 * 128 * 2.4
 # plain copy of known size (FETCH_SIZE counts half the bytes read, WRITE_SIZE
 # the bytes written: the calibration in profiles/n64800_state_kernels_bench.md).
 MEASURED_TRAFFIC_PER_FI = {"layered_stair": 1036154, "layered_general": 1832398, "check": 1201488,
-                           "variable": 1477744}
+                           "variable": 1477744, "frame": 1826000}
 # Vector-ALU issue: 256 CUs x 4 SIMDs, one 64-lane FP32/INT32 instruction per
 # SIMD every 4 clocks (16 lanes per clock) at 2.4 GHz; wave-level VALU
 # instructions per frame-iteration measured with rocprofv3 SQ_INSTS_VALU on
@@ -243,7 +243,7 @@ def main():
         prof = None
         if profile:
             prof = {}
-            for k, name in enumerate(["check", "variable", "syndrome", "layered"]):
+            for k, name in enumerate(["check", "variable", "syndrome", "layered", "frame"]):
                 ms, la, fi = ctypes.c_double(), ctypes.c_uint64(), ctypes.c_uint64()
                 lib.gf2l_profile_read_kernel(ctx.handle, k, ctypes.byref(ms), ctypes.byref(la), ctypes.byref(fi))
                 prof[name] = (ms.value, la.value, fi.value)
@@ -299,11 +299,15 @@ def main():
     #   layered, general kernel: HBM: 24M, read and write the beliefs of block-columns outside LDS
     #             once per edge (8 E_glob) and read them once for the hard decisions (4 z (nb - X));
     #             LDS: the same for the X columns in LDS
+    #   frame     plain BP, one workgroup per frame: read and write the 12-byte state of every check (24M),
+    #             read the LLRs (4N), read and write the beliefs (8N)
     per_fi = {"check": 4 * cv_n + 24 * M, "variable": 12 * M + 8 * cv_n + cv_n // 8, "syndrome": cv_n // 8,
+              "frame": 24 * M + 12 * cv_n,
               "layered": (24 * M + 8 * z * (nb - kb)) if stair else
                          (24 * M + 8 * (E - edges_lds) + 4 * z * (nb - X))}
     lds_per_fi = 8 * edges_lds + 4 * z * X
     kernels = {"check": "cn_state_kernel", "variable": "vn_state_kernel", "syndrome": "syn_words_kernel",
+               "frame": "flood_kernel",
                "layered": "lnms_stair_kernel" if stair else "lnms_fwd_kernel"}
     traffic_key = {"layered": "layered_stair" if stair else "layered_general"}
 

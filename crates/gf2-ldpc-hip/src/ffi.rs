@@ -38,6 +38,7 @@ pub const GF2L_KERNEL_CHECK: c_int = 0;
 pub const GF2L_KERNEL_VARIABLE: c_int = 1;
 pub const GF2L_KERNEL_SYNDROME: c_int = 2;
 pub const GF2L_KERNEL_LAYERED: c_int = 3;
+pub const GF2L_KERNEL_FRAME: c_int = 4;
 
 pub const GF2L_PROFILE_ALL: c_int = 1;
 pub const GF2L_PROFILE_LAYERED: c_int = 2;
@@ -59,6 +60,7 @@ pub const GF2L_TUNE_LAYERED_COLUMNS: c_int = 5;
 pub const GF2L_TUNE_LAYERED_KERNEL: c_int = 6;
 pub const GF2L_TUNE_LDS_GROUPS: c_int = 7;
 pub const GF2L_TUNE_HBM_GRAPH: c_int = 8;
+pub const GF2L_TUNE_FRAME_KERNEL: c_int = 9;
 
 pub const GF2L_NOALLOC_SCRATCH_BYTES: u32 = 64 << 20;
 

@@ -36,12 +36,14 @@ TUNE_LAYERED_COLUMNS = 5
 TUNE_LAYERED_KERNEL = 6
 TUNE_LDS_GROUPS = 7
 TUNE_HBM_GRAPH = 8
+TUNE_FRAME_KERNEL = 9
 LAYERED_AUTO, LAYERED_GENERAL, LAYERED_STAIRCASE = 0, 1, 2
 
 KERNEL_CHECK = 0
 KERNEL_VARIABLE = 1
 KERNEL_SYNDROME = 2
 KERNEL_LAYERED = 3
+KERNEL_FRAME = 4
 PROFILE_ALL = 1
 PROFILE_LAYERED = 2
 

@@ -542,6 +542,35 @@ __device__ __forceinline__ uint64_t cyc64(const uint64_t *v, uint32_t z, uint32_
     return r;
 }
 
+// Barrier that orders LDS accesses only: loads and stores to global memory in
+// flight are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// LDS pointers typed as such, so every access is a ds_ instruction (a
+// generic pointer held in a struct compiles to flat accesses, which count
+// against the vector-memory counter and would wait for the loads ahead).
+typedef __attribute__((address_space(3))) float lds_float;
+typedef __attribute__((address_space(3))) uint64_t lds_u64;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+
+// LDS word at a byte address.
+__device__ __forceinline__ float lds_ld(uint32_t addr) { return *(const lds_float *)(size_t)addr; }
+__device__ __forceinline__ void lds_st(uint32_t addr, float v) { *(lds_float *)(size_t)addr = v; }
+
+// cyc64 over words in LDS.
+__device__ __forceinline__ uint64_t cyc64_lds(const lds_u64 *v, uint32_t z, uint32_t zw, uint32_t pos) {
+    const uint32_t wi = pos >> 6, sh = pos & 63u;
+    uint64_t r = v[wi] >> sh;
+    if (sh && wi + 1 < zw) r |= v[wi + 1] << (64u - sh);
+    const uint32_t avail = z - pos;
+    if (avail < 64u) r |= v[0] << avail;
+    return r;
+}
+
 // Returns nonzero (uniform over the workgroup) when a check is unsatisfied
 // by the frame's nb*zw hard-decision words in sh (LDS, complete and visible
 // to the whole workgroup).

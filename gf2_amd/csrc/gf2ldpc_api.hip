@@ -99,6 +99,76 @@ int resolve_path(const gf2l_ctx *ctx, const gf2l::CodeView &cv) {
     }
 }
 
+// Whether a plain batch of F frames runs the whole-frame kernel.
+static bool use_frame_kernel(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F) {
+    if (!code->flood.nd || ctx->tune.frame_kernel == 1) return false;
+    if (ctx->tune.frame_kernel == 2) return true;
+    if (ctx->path != gf2l::kAuto || ctx->tune.hbm_graph) return false;
+    // A frame of the whole-frame kernel has one workgroup and a compute unit's
+    // rate; the STATE kernels spread a frame over the chip but pay four
+    // launches an iteration (30 to 40 us).  Codes of which two workgroups fit a
+    // compute unit (N = 16200) win from one frame on (364 -> 175 us at rate
+    // 0.44, 987 -> 463 us at rate 2/3).  Longer ones win once the STATE
+    // kernels' iteration takes longer than a workgroup's 53 us (N = 64800, r
+    // 1/2: 1671 -> 1629 us at 48 frames, 1555 -> 1575 us at 32), those whose
+    // columns exceed the LDS later (r 2/3: 2514 -> 2387 us at 100, 1.28x at
+    // 160; r 5/6: 0.92x at 160).
+    const CodeView &cv = code->view;
+    if (flood_bytes(cv, code->flood) <= 80 * 1024) return true;
+    const uint32_t cus = (uint32_t)ctx->num_cus;
+    return F >= (code->flood.X == cv.nb - cv.mb ? cus / 6 : cus * 3 / 4);
+}
+
+// Plain min-sum by the whole-frame kernel (flood.hip): results of every frame
+// but those in `left` (an LLR or belief too large for it).
+static int decode_flood(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
+                        uint64_t *d_msg, uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd,
+                        std::vector<uint32_t> &left) {
+    const CodeView &cv = code->view;
+    hipStream_t s = ctx->stream;
+    const uint32_t grid = flood_grid(cv, code->flood, F, ctx->num_cus);
+    int rc = ensure_buffers(ctx, F, 0, 3ull * cv.m * grid, ((size_t)cv.n + cv.n - cv.m) * grid, 0, 0);
+    if (rc != GF2L_OK) return rc;
+    Workspace &ws = ctx->ws;
+    GF2L_HIP(ctx, launch_clear_words(ws.counts, 4, s));
+    FloodArgs a{};
+    a.cv = cv;
+    a.plan = code->flood;
+    a.llr = d_llr;
+    a.frames = F;
+    a.max_it = max_it;
+    a.state = ws.state;
+    a.bel = ws.belief;
+    a.ctr = ws.counts + 2;
+    a.list = ws.lists;
+    a.count = ws.counts;
+    a.msg = d_msg;
+    a.iters = d_iters;
+    a.conv = d_conv;
+    a.synd = d_synd;
+    Profile &pf = ctx->prof;
+    const bool timed = pf.on && pf.all;
+    if (timed) GF2L_HIP(ctx, hipEventRecord(pf.lev[0], s));
+    GF2L_HIP(ctx, launch_flood(a, grid, s));
+    if (timed) GF2L_HIP(ctx, hipEventRecord(pf.lev[1], s));
+    GF2L_HIP(ctx, hipMemcpyAsync(ws.h_count, ws.counts, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    GF2L_HIP(ctx, hipStreamSynchronize(s));
+    if (timed) {
+        float ms = 0.0f;
+        GF2L_HIP(ctx, hipEventElapsedTime(&ms, pf.lev[0], pf.lev[1]));
+        pf.ms[4] += ms;
+        pf.launches[4] += 1;
+        pf.whole_frame_iters += ws.h_count[3];
+    }
+    left.resize(ws.h_count[0]);
+    if (!left.empty()) {
+        GF2L_HIP(ctx, hipMemcpyAsync(left.data(), ws.lists, left.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        GF2L_HIP(ctx, hipStreamSynchronize(s));
+        std::sort(left.begin(), left.end());
+    }
+    return GF2L_OK;
+}
+
 // Runs the decoder on device buffers.  Without weights: plain min-sum for up
 // to max_it iterations.  With weights d_w ([max_it][nbe]): max_it weighted
 // iterations, then frames still failing the syndrome get up to fb_it plain
@@ -164,6 +234,13 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         }
         return GF2L_OK;
     }
+    std::vector<uint32_t> left;  // frames the whole-frame kernel leaves to the general ones
+    bool whole = false;
+    if (path == gf2l::kState && !d_w && !d_fb && !h_trace_c2v && use_frame_kernel(ctx, code, F)) {
+        const int rcf = decode_flood(ctx, code, d_llr, F, max_it, d_msg, d_iters, d_conv, d_synd, left);
+        if (rcf != GF2L_OK || left.empty()) return rcf;
+        whole = true;
+    }
     int rc = ensure_workspace(ctx, cv, path, F);
     if (rc != GF2L_OK) return rc;
     gf2l::Workspace &ws = ctx->ws;
@@ -177,7 +254,7 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         ~Free() { hipFree(a); hipFree(b); }
     } free_trace{d_tc, d_tb};
     return run_hbm(ctx, cv, path, ws, d_llr, F, max_it, d_w, fb_it, fb_continue, d_msg, d_iters, d_conv,
-                   d_synd, d_fb, h_trace_c2v, h_trace_bel, trace_iters, d_tc, d_tb);
+                   d_synd, d_fb, h_trace_c2v, h_trace_bel, trace_iters, d_tc, d_tb, true, whole ? &left : nullptr);
 }
 
 // Captures `unroll` (even) plain iterations of the final phase as a graph:
@@ -242,7 +319,8 @@ int hbm_graph(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const 
 int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const float *d_llr, uint32_t F,
             uint32_t max_it, const float *d_w, uint32_t fb_it, bool fb_continue, uint64_t *d_msg,
             uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd, uint8_t *d_fb, float *h_trace_c2v,
-            float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs) {
+            float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs,
+            const std::vector<uint32_t> *only) {
     hipStream_t s = ctx->stream;
     const size_t E = (size_t)cv.nbe * cv.z;
     gf2l::Profile &pf = ctx->prof;
@@ -256,6 +334,12 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
     const bool ph = pf.on && pf.all;  // time these launches
     const bool use_graph = graphs && ctx->tune.hbm_graph && !h_trace_c2v && !ph;
     uint32_t running = F;  // frames entering the first iteration of the current batch
+    if (only) {
+        running = (uint32_t)only->size();
+        GF2L_HIP(ctx, hipMemcpyAsync(ws.lists, only->data(), running * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+        GF2L_HIP(ctx, hipMemcpyAsync(ws.counts, &running, sizeof(uint32_t), hipMemcpyHostToDevice, s));
+        GF2L_HIP(ctx, hipStreamSynchronize(s));
+    }
     uint32_t queued = 0;   // iterations enqueued since the last readback
     // per-kernel times of the iterations of one batch (stream synchronized)
     auto collect = [&](uint32_t iters) -> int {
@@ -580,12 +664,13 @@ int gf2l_profile_enable(gf2l_ctx *ctx, int on) {
             for (auto &e : pf.ev) GF2L_HIP(ctx, hipEventCreate(&e));
             for (auto &e : pf.lev) GF2L_HIP(ctx, hipEventCreate(&e));
         }
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < 5; ++k) {
             pf.ms[k] = 0;
             pf.launches[k] = 0;
         }
         pf.frame_iters = 0;
         pf.layered_frame_iters = 0;
+        pf.whole_frame_iters = 0;
         pf.on = on != 0;
         pf.all = on != GF2L_PROFILE_LAYERED;
         return GF2L_OK;
@@ -604,11 +689,14 @@ int gf2l_profile_read(gf2l_ctx *ctx, double *ms, uint64_t *launches, uint64_t *f
 
 int gf2l_profile_read_kernel(gf2l_ctx *ctx, int kernel, double *ms, uint64_t *launches,
                              uint64_t *frame_iterations) {
-    if (!ctx || kernel < 0 || kernel > GF2L_KERNEL_LAYERED) return GF2L_ERR_INVALID;
+    if (!ctx || kernel < 0 || kernel > GF2L_KERNEL_FRAME) return GF2L_ERR_INVALID;
     const gf2l::Profile &pf = ctx->prof;
     if (ms) *ms = pf.ms[kernel];
     if (launches) *launches = pf.launches[kernel];
-    if (frame_iterations) *frame_iterations = kernel == GF2L_KERNEL_LAYERED ? pf.layered_frame_iters : pf.frame_iters;
+    if (frame_iterations)
+        *frame_iterations = kernel == GF2L_KERNEL_LAYERED ? pf.layered_frame_iters
+                            : kernel == GF2L_KERNEL_FRAME ? pf.whole_frame_iters
+                                                          : pf.frame_iters;
     return GF2L_OK;
 }
 
@@ -772,6 +860,10 @@ int gf2l_set_tuning(gf2l_ctx *ctx, int key, int value) {
                 if (value < 0 || value > 1) return fail(ctx, GF2L_ERR_INVALID, "hbm graph out of [0,1]");
                 ctx->tune.hbm_graph = value;
                 return GF2L_OK;
+            case GF2L_TUNE_FRAME_KERNEL:
+                if (value < 0 || value > 2) return fail(ctx, GF2L_ERR_INVALID, "frame kernel out of [0,2]");
+                ctx->tune.frame_kernel = value;
+                return GF2L_OK;
             case GF2L_TUNE_LDS_GROUPS:
                 if (value < 0 || value > 512) return fail(ctx, GF2L_ERR_INVALID, "lds groups out of [0,512]");
                 ctx->tune.lds_groups = value;
@@ -815,8 +907,13 @@ int gf2l_code_qc(gf2l_ctx *ctx, uint32_t mb, uint32_t nb, uint32_t z, const int3
             }
             c->h_row_ptr[br + 1] = (uint32_t)c->h_row_edge.size();
         }
-        const int rc = gf2l::build_qc_view(ctx, c, mb, nb, z, 0);
+        int rc = gf2l::build_qc_view(ctx, c, mb, nb, z, 0);
         if (rc != GF2L_OK) return rc;
+        rc = gf2l::build_flood_plan(ctx, c);
+        if (rc != GF2L_OK) {
+            gf2l_code_destroy(c);
+            return rc;
+        }
         *out = c;
         return GF2L_OK;
     });
@@ -837,6 +934,7 @@ void gf2l_code_destroy(gf2l_code *code) {
     if (!code) return;
     hipSetDevice(code->device);
     hipFree(code->d_tables);
+    hipFree(code->d_flood);
     delete code;
 }
 

@@ -45,6 +45,18 @@ struct CodeView {
     uint32_t dvb_kb = 0, dvb_q = 0;
 };
 
+// Row tables of the whole-frame flooding kernel (flood.hip) for a staircase
+// quasi-cyclic code; nd == 0: the code lacks the structure.
+struct FloodPlan {
+    const uint2 *edge = nullptr;    // [mb][nd] information inputs of a block-row: {4 * (column * z + shift), z - shift}
+    const uint32_t *row = nullptr;  // [mb] information inputs | those accumulated in LDS << 8 | degree of the state layout << 16
+    const uint32_t *xptr = nullptr; // [kb-X+1] into xedge
+    const uint2 *xedge = nullptr;   // edges of the information columns past X: {byte offset of the block-row's
+                                    // states, shift | position << 16 | shift of its sign bit << 24}
+    uint32_t nd = 0;                // information inputs per row of the instantiation (rows padded to it)
+    uint32_t X = 0;                 // information block-columns accumulated in LDS
+};
+
 // Device view of a general sparse code (LdpcCode::from_edges): CSR rows with
 // ascending columns and, per variable, its CSR edges in ascending check
 // order (the stable transpose of SpBitMatrix::transpose).
@@ -86,11 +98,12 @@ struct Profile {
     bool on = false;
     bool all = true;                  // every launch; false: the layered kernel only
     hipEvent_t ev[4 * kProfileSlots] = {};
-    hipEvent_t lev[2] = {};           // around the layered kernel
-    double ms[4] = {0, 0, 0, 0};      // check, variable, syndrome, layered kernels
-    uint64_t launches[4] = {0, 0, 0, 0};
+    hipEvent_t lev[2] = {};           // around the layered or the whole-frame kernel
+    double ms[5] = {};                // check, variable, syndrome, layered, whole-frame kernels
+    uint64_t launches[5] = {};
     uint64_t frame_iters = 0;         // sum over HBM-path launches of frames processed
     uint64_t layered_frame_iters = 0; // layered iterations run, summed over frames
+    uint64_t whole_frame_iters = 0;   // iterations of the whole-frame kernel, summed over frames
 };
 
 // Launch-shape tunables of the HBM paths (set by gf2l_set_tuning or the
@@ -104,6 +117,7 @@ struct Tuning {
     int layered_kernel = 0; // 0: staircase kernel where it applies, 1: general kernel, 2: staircase kernel
     int lds_groups = 0;  // thread groups per workgroup of the LDS path (0: automatic)
     int hbm_graph = 0;   // 1: plain iterations of the HBM paths replayed from a captured graph
+    int frame_kernel = 0; // whole-frame flooding kernel: 0 automatic, 1 never, 2 wherever the code allows it
 };
 
 // Word offset of the item counters in Workspace::counts and its size (two
@@ -159,6 +173,21 @@ struct LayeredArgs {
     uint64_t stair_sync[4];  // staircase kernel: bit r set when a barrier must follow block-row r
 };
 
+// Arguments of the whole-frame flooding kernel (flood.hip).
+struct FloodArgs {
+    CodeView cv;
+    FloodPlan plan;
+    const float *llr;        // [frames][n]
+    uint32_t frames, max_it;
+    uint32_t *state;         // per workgroup [mb][z][3] check states
+    float *bel;              // per workgroup [kb][z] and [nb][z] beliefs
+    uint32_t *ctr;           // [0] next frame, [1] iterations run, summed over frames (zeroed before the launch)
+    uint32_t *list, *count;  // frames left to the general kernels (count zeroed before the launch)
+    uint64_t *msg;
+    uint32_t *iters;
+    uint8_t *conv, *synd;
+};
+
 // Arguments of the layered backward kernel (layered.hip).
 struct LayeredBwdArgs {
     CodeView cv;
@@ -186,6 +215,8 @@ struct gf2l_code {
     std::vector<uint2> h_row_edge, h_col_edge;
     std::vector<uint4> h_col_info;
     void *d_tables = nullptr;    // one allocation backing the view's tables
+    gf2l::FloodPlan flood;       // whole-frame flooding kernel (d_flood backs its tables)
+    void *d_flood = nullptr;
     int device = 0;
 };
 
@@ -276,11 +307,13 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
 // Iteration loop of the HBM paths (STATE / STREAM) over a workspace the
 // caller has prepared (gf2ldpc_api.hip); allocates nothing.  Used by
 // decode_device after growing the context's workspace and by the
-// no-allocation entry point over its static scratch array.
+// no-allocation entry point over its static scratch array.  only (may be
+// null): the frames to decode, of the F the buffers hold.
 int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const float *d_llr, uint32_t F,
             uint32_t max_it, const float *d_w, uint32_t fb_it, bool fb_continue, uint64_t *d_msg,
             uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd, uint8_t *d_fb, float *h_trace_c2v,
-            float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs = true);
+            float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs = true,
+            const std::vector<uint32_t> *only = nullptr);
 // Decoder path (GF2L_PATH_*) the context would run a quasi-cyclic code on,
 // or -1 when a forced path cannot run it.
 int resolve_path(const gf2l_ctx *ctx, const CodeView &cv);
@@ -319,6 +352,15 @@ hipError_t launch_layered_bwd(const LayeredBwdArgs &a, int num_cus, hipStream_t 
 size_t layered_stair_bytes(const CodeView &cv);
 uint32_t layered_stair_degree(const gf2l_code *code, uint64_t *deg_mask = nullptr, uint64_t *sync_mask = nullptr);
 hipError_t launch_layered_stair(const LayeredArgs &a, uint32_t dh, int num_cus, hipStream_t s);
+
+// Whole-frame flooding kernel (flood.hip): builds the row tables of a
+// quasi-cyclic code that has the structure (leaves code->flood empty
+// otherwise), its dynamic LDS, workgroups for a batch, and the launcher.
+int build_flood_plan(gf2l_ctx *ctx, gf2l_code *c);
+size_t flood_bytes(const CodeView &cv, const FloodPlan &pl);
+hipError_t launch_clear_words(uint32_t *words, uint32_t count, hipStream_t s);
+uint32_t flood_grid(const CodeView &cv, const FloodPlan &pl, uint32_t frames, int num_cus);
+hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s);
 
 // Plain min-sum on a general sparse code (csr.hip).
 int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,

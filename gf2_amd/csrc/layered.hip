@@ -229,19 +229,6 @@ __global__ void __launch_bounds__(512) lnms_fwd_kernel(LayeredArgs a) {
 // unused global row of block-column kb-1, every block-row its column kb+r
 // as it stands; the information rows are rewritten at hand-over).
 
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// LDS pointers typed as such, so every access is a ds_ instruction (a
-// generic pointer held in a struct compiles to flat accesses, which count
-// against the vector-memory counter and would wait for the loads ahead).
-typedef __attribute__((address_space(3))) float lds_float;
-typedef __attribute__((address_space(3))) uint64_t lds_u64;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-
 struct StairFrame {
     lds_u64 *hb;       // [nb][zw] hard decisions
     const lds_u32 *tab; // [nbe][4] per edge: LDS byte address of its column's
@@ -252,8 +239,6 @@ struct StairFrame {
     uint32_t kb, i;    // i = threadIdx.x < z
 };
 
-__device__ __forceinline__ float lds_ld(uint32_t addr) { return *(const lds_float *)(size_t)addr; }
-__device__ __forceinline__ void lds_st(uint32_t addr, float v) { *(lds_float *)(size_t)addr = v; }
 // x * (-1)^s for s in {0, 1}: a sign flip, exact
 __device__ __forceinline__ float flip(float x, uint32_t s) { return __uint_as_float(__float_as_uint(x) ^ (s << 31)); }
 
@@ -355,17 +340,8 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
 }
 
 // Parity checks over the hard-decision words, the code's edge tables read
-// from LDS copies (rp, re); uniform over the workgroup.
-__device__ __forceinline__ uint64_t cyc64_lds(const lds_u64 *v, uint32_t z, uint32_t zw, uint32_t pos) {
-    const uint32_t wi = pos >> 6, sh = pos & 63u;
-    uint64_t r = v[wi] >> sh;
-    if (sh && wi + 1 < zw) r |= v[wi + 1] << (64u - sh);
-    const uint32_t avail = z - pos;
-    if (avail < 64u) r |= v[0] << avail;
-    return r;
-}
-
-// The staircase kernel runs z threads (zw waves): the block size comes from
+// from LDS copies (rp, re); uniform over the workgroup.  The staircase
+// kernel runs z threads (zw waves): the block size comes from
 // the code view (a scalar), not from the dispatch packet (a vector load,
 // whose wait would also wait for every load ahead).
 __device__ __forceinline__ uint32_t stair_unsat(const CodeView &cv, const lds_u64 *sh, const lds_u32 *rp,

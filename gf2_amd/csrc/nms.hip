@@ -401,10 +401,6 @@ int layered_forward_backward(gf2l_ctx *ctx, gf2l_nms *q, const float *d_llr, con
     return GF2L_OK;
 }
 
-__global__ void clear_words_kernel(uint32_t *p, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
-}
-
 // Layered decode: the layered kernel over all frames (early stop after any
 // iteration), then plain flooding min-sum continued from the layered state
 // for the frames it handed over, up to fb_it iterations (reported as T + u;
@@ -422,8 +418,7 @@ int layered_decode(gf2l_ctx *ctx, const gf2l_nms *q, const float *d_llr, uint32_
     Profile &pf = ctx->prof;
     hipStream_t s = ctx->stream;
     // running counts, item counters and the layered frame counters start at zero
-    hipLaunchKernelGGL(clear_words_kernel, dim3((kCountsWords + 255) / 256), dim3(256), 0, s, ws.counts, kCountsWords);
-    GF2L_HIP(ctx, hipGetLastError());
+    GF2L_HIP(ctx, launch_clear_words(ws.counts, kCountsWords, s));
     LayeredArgs a{};
     a.cv = cv;
     a.llr = d_llr;

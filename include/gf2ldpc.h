@@ -65,7 +65,8 @@ void *gf2l_stream(gf2l_ctx *ctx);
 /* Per-kernel timing: HIP events are recorded around kernel launches on the
  * context's stream.  on = GF2L_PROFILE_ALL (or any value other than 0 and
  * GF2L_PROFILE_LAYERED): every check / variable / syndrome launch of the HBM
- * paths and every layered learned-decoder launch; the HBM paths then read the
+ * paths, every whole-frame launch and every layered learned-decoder launch; the
+ * HBM paths then read the
  * running count back after every iteration (frames processed per launch).
  * on = GF2L_PROFILE_LAYERED: the layered kernel only, so the plain
  * continuation after it runs as it does unprofiled.  0: off.  Enabling (or
@@ -80,12 +81,13 @@ int gf2l_profile_enable(gf2l_ctx *ctx, int on);
 int gf2l_profile_read(gf2l_ctx *ctx, double *ms, uint64_t *launches, uint64_t *frame_iterations);
 /* One kernel's figures: summed ms, launches, and frame-iterations processed
  * (for the check / variable / syndrome kernels the HBM paths' frames summed
- * over iterations, for the layered learned decoder's kernel its iterations
- * summed over frames). */
+ * over iterations, for the layered learned decoder's kernel and the
+ * whole-frame flooding kernel their iterations summed over frames). */
 #define GF2L_KERNEL_CHECK 0
 #define GF2L_KERNEL_VARIABLE 1
 #define GF2L_KERNEL_SYNDROME 2
 #define GF2L_KERNEL_LAYERED 3
+#define GF2L_KERNEL_FRAME 4
 int gf2l_profile_read_kernel(gf2l_ctx *ctx, int kernel, double *ms, uint64_t *launches,
                              uint64_t *frame_iterations);
 
@@ -97,6 +99,8 @@ int gf2l_profile_read_kernel(gf2l_ctx *ctx, int kernel, double *ms, uint64_t *la
  *                     edge (check degree <= 32)
  *   GF2L_PATH_STATE   per-iteration kernels over HBM, 12-byte compressed
  *                     state per check from which messages are rebuilt
+ * Where AUTO picks STATE for a staircase quasi-cyclic code, plain decodes of
+ * enough frames run a whole-frame kernel instead (GF2L_TUNE_FRAME_KERNEL).
  * A forced path that cannot run a code makes decode calls return
  * GF2L_ERR_UNSUPPORTED.  All paths give identical results. */
 #define GF2L_PATH_AUTO 0
@@ -178,7 +182,12 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
  *                        batch size and buffers and kept by the context;
  *                        0 (default): launched one by one.  Never while
  *                        profiling or tracing, never by the no-allocation
- *                        entry point. */
+ *                        entry point.
+ *   GF2L_TUNE_FRAME_KERNEL plain decodes of staircase quasi-cyclic codes on
+ *                        the STATE path: 0 (default) one workgroup per frame
+ *                        for all its iterations where that is faster (never
+ *                        on a forced path), 1 never, 2 wherever the code has
+ *                        the structure. */
 #define GF2L_TUNE_WG_PER_CU 1
 #define GF2L_TUNE_XCD_MAP 2
 #define GF2L_TUNE_GRAPH_ITERS 3
@@ -187,6 +196,7 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
 #define GF2L_TUNE_LAYERED_KERNEL 6
 #define GF2L_TUNE_LDS_GROUPS 7
 #define GF2L_TUNE_HBM_GRAPH 8
+#define GF2L_TUNE_FRAME_KERNEL 9
 int gf2l_set_tuning(gf2l_ctx *ctx, int key, int value);
 
 /* ---- codes ------------------------------------------------------------ */

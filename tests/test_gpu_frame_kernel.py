@@ -1,0 +1,92 @@
+"""The whole-frame flooding kernel against the oracle: one workgroup per frame
+on staircase quasi-cyclic codes, bit-exact, over the shapes where its row
+tables, wave layout and LDS split differ."""
+import numpy as np
+import pytest
+
+from gf2_amd import _lib, codes
+from gf2_amd.ldpc import Context, LdpcCode, QuasiCyclicLdpc, decode_batch_arrays, qc_ira_base_matrix
+from oracle import oracle as orc
+from tests import frames
+
+pytestmark = pytest.mark.gpu
+
+# (mb, nb, z, information column weights, Eb/N0)
+SHAPES = {
+    "two-rows-one-wave": (2, 5, 64, [2, 2, 1], 4.0),
+    "odd-rows-ragged-lift": (3, 9, 100, [3, 3, 2, 2, 2, 1], 4.0),
+    "short-lift-96": (12, 24, 96, [6] * 4 + [3] * 8, 2.2),
+    "largest-lift": (7, 20, 384, [4] * 5 + [3] * 8, 3.0),
+    "few-heavy-columns": (10, 14, 320, [10, 9, 5, 2], 2.0),
+    "degree-25-columns-past-lds": (5, 120, 360, [1] * 115, 6.0),
+    "columns-past-lds": (40, 160, 360, [7] * 30 + [3] * 90, 3.0),
+    "lift-above-the-kernel": (6, 15, 400, [3] * 9, 3.0),  # runs the general kernels
+}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    orc.build()
+    return Context(0)
+
+
+def decode(ctx, code, llr, max_it, mode):
+    ctx.set_tuning(_lib.TUNE_FRAME_KERNEL, mode)
+    try:
+        return decode_batch_arrays(code, llr, max_it)
+    finally:
+        ctx.set_tuning(_lib.TUNE_FRAME_KERNEL, 0)
+
+
+def same(a, b, what):
+    for name, x, y in zip(["msg", "iterations", "converged", "syndrome_ok"], a, b):
+        assert np.array_equal(x, y), f"{what}: {name} differs at {np.nonzero(np.asarray(x) != y)[0][:8]}"
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_matches_oracle(ctx, shape):
+    mb, nb, z, weights, ebn0 = SHAPES[shape]
+    base = qc_ira_base_matrix(5, mb, nb, z, weights)
+    code = LdpcCode(QuasiCyclicLdpc(base, z), ctx)
+    oc = orc.Code.from_qc(base, z)
+    F = 6 if nb * z > 30000 else 37
+    _, _, llr = frames.random_frames(base, z, F, ebn0, seed=11)
+    rng = np.random.default_rng(12)
+    llr[rng.random(llr.shape) < 0.002] = -0.0
+    llr[rng.random(llr.shape) < 0.002] = 0.0
+    llr[-1] = rng.normal(0, 1, llr.shape[1]).astype(np.float32)  # no codeword near: runs every iteration
+    for count, max_it in ((1, 20), (F, 1), (F, 2), (F, 20)):
+        print("[gpu-case] frame kernel", shape, count, max_it, flush=True)
+        same(decode(ctx, code, llr[:count], max_it, 2), oc.decode_batch(llr[:count], max_it, threads=8),
+             f"{shape} {count}x{max_it}")
+
+
+def test_more_frames_than_workgroups(ctx):
+    """Frames are drawn from a counter: each workgroup decodes several."""
+    spec = codes.QcIraSpec(16200, 7200, 360)
+    base = spec.base_matrix()
+    code = LdpcCode(QuasiCyclicLdpc(base, spec.z), ctx)
+    _, _, llr = frames.random_frames(base, spec.z, 24, 2.6, seed=3)
+    print("[gpu-case] frame kernel, 1200 frames", flush=True)
+    ref = orc.Code.from_qc(base, spec.z).decode_batch(llr, 50, threads=8)
+    got = decode(ctx, code, np.tile(llr, (50, 1)), 50, 0)
+    same(got, [np.tile(r, (50, 1)) if r.ndim == 2 else np.tile(r, 50) for r in ref], "tiled")
+
+
+def test_frames_it_leaves_to_the_general_kernels(ctx):
+    """Infinite, NaN and very large LLRs: those frames come out as the general
+    kernels decode them, the others as ever."""
+    spec = codes.QcIraSpec(16200, 7200, 360)
+    base = spec.base_matrix()
+    code = LdpcCode(QuasiCyclicLdpc(base, spec.z), ctx)
+    _, _, llr = frames.random_frames(base, spec.z, 12, 2.4, seed=4)
+    rng = np.random.default_rng(5)
+    for f, v in ((1, np.inf), (4, -np.inf), (7, np.nan), (9, 2e30), (10, -3.3e38)):
+        llr[f, rng.integers(0, spec.n, 9)] = v
+    llr[11] *= np.float32(1e28)  # beliefs pass the limit while it iterates
+    print("[gpu-case] frame kernel, special LLRs", flush=True)
+    got = decode(ctx, code, llr, 50, 2)
+    same(got, decode(ctx, code, llr, 50, 1), "special")
+    finite = [f for f in range(12) if np.isfinite(llr[f]).all()]
+    ref = orc.Code.from_qc(base, spec.z).decode_batch(llr[finite], 50, threads=8)
+    same([r[finite] for r in got], ref, "finite")
