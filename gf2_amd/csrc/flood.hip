@@ -61,6 +61,10 @@ namespace {
 constexpr uint32_t kFloodGroups = 2;
 constexpr uint32_t kFloodThreads = 768;  // two groups of up to 384 lanes
 constexpr float kFloodLimit = 1e30f;
+// Information inputs per row of the instantiations.
+#define GF2L_FLOOD_DEGREES                                                                              \
+    GF2L_FLOOD(4) GF2L_FLOOD(5) GF2L_FLOOD(6) GF2L_FLOOD(8) GF2L_FLOOD(9) GF2L_FLOOD(10) GF2L_FLOOD(11) \
+    GF2L_FLOOD(13) GF2L_FLOOD(15) GF2L_FLOOD(17) GF2L_FLOOD(21) GF2L_FLOOD(25)
 
 __device__ __forceinline__ bool too_large(float v) { return !(fabsf(v) < kFloodLimit); }
 
@@ -172,10 +176,11 @@ __device__ __forceinline__ uint3 flood_check(const FloodIn<ND> &in, uint32_t nin
 // LDS of one workgroup.
 struct FloodLds {
     lds_float *acc;      // [X][z] beliefs being formed
-    lds_float *carry;    // [4][lanes] L + message of the row above, parity columns
+    lds_float *carry;    // [4][lanes] L + message of the row above, parity columns; one unused row
     lds_u64 *hb;         // [nb][zw] hard decisions
     lds_u32 *chk;        // nbe: hard-decision word of the block-column | shift << 16
     lds_u32 *rp;         // mb + 1
+    uint32_t unused;     // this lane's byte offset of the unused row from acc
     lds_u32 *done, *bad; // rows added (waves); per wave: unsatisfied | too large << 1
 };
 
@@ -201,16 +206,16 @@ __device__ __forceinline__ void stb(T *base, uint32_t off, T v) {
 // float atomic (ds_add_f32) would need no order within the row, but measured
 // three times slower for the whole kernel (96 ms against 30 ms per 4096-frame
 // batch of the N=64800 code).
-template <int NI, bool ALL>
+template <int NI, bool GUARD>
 __device__ __forceinline__ void flood_add(lds_float *acc, const uint32_t *ad, const float *c, uint32_t nlds) {
     auto at = [&](int p) { return (lds_float *)((__attribute__((address_space(3))) char *)acc + ad[p]); };
     float v[NI];
 #pragma unroll
     for (int p = 0; p < NI; ++p)
-        if (ALL || p < (int)nlds) v[p] = *at(p);
+        if (!GUARD || p < (int)nlds) v[p] = *at(p);
 #pragma unroll
     for (int p = 0; p < NI; ++p)
-        if (ALL || p < (int)nlds) *at(p) = v[p] + c[p];
+        if (!GUARD || p < (int)nlds) *at(p) = v[p] + c[p];
 }
 
 // Hard-decision word of a column from its final beliefs (one per lane);
@@ -249,10 +254,17 @@ __device__ __forceinline__ uint64_t flood_row(const FloodFrame &F, const FloodIn
     float prev = 0.0f;
     if (F.act) {
         prev = *above;
-        if (!GENERAL && (!EXTRA || nlds == (uint32_t)NI))
+        if constexpr (GENERAL) {
             flood_add<NI, true>(F.S.acc, ad, c, nlds);
-        else
+        } else {
+            // messages to columns past the LDS go to an unused row: a select
+            // each, where a branch each split the row's reads and writes
+            if constexpr (EXTRA) {
+#pragma unroll
+                for (int p = 0; p < NI; ++p) ad[p] = p < (int)nlds ? ad[p] : F.S.unused;
+            }
             flood_add<NI, false>(F.S.acc, ad, c, nlds);
+        }
         *slot = own;
     }
     // a wave's LDS operations complete in order: the count lands after the adds
@@ -429,32 +441,46 @@ __device__ __forceinline__ uint32_t flood_frame(FloodFrame &F, uint32_t max_it, 
     }
 }
 
+// LDS layout of a workgroup for one code, and the copy of its parity checks.
+__device__ __forceinline__ FloodLds flood_lds(const CodeView &cv, const FloodPlan &pl, uint64_t *smem,
+                                              uint32_t *done, uint32_t *bad) {
+    FloodLds S;
+    S.acc = (lds_float *)smem;  // first: its address folds into the offsets of the accesses
+    S.hb = (lds_u64 *)(S.acc + ((pl.X * cv.z + 1u) & ~1u));
+    S.carry = (lds_float *)(S.hb + cv.nb * cv.zw);
+    const uint32_t lanes = blockDim.x / kFloodGroups;
+    S.chk = (lds_u32 *)(S.carry + 5u * lanes);
+    S.rp = S.chk + cv.nbe;
+    S.unused = (uint32_t)((size_t)S.carry - (size_t)S.acc) + 4u * (4u * lanes + threadIdx.x % lanes);
+    S.done = (lds_u32 *)done;
+    S.bad = (lds_u32 *)bad;
+    for (uint32_t e = threadIdx.x; e < cv.nbe; e += blockDim.x) {
+        const uint2 r = cv.row_edge[e];
+        S.chk[e] = r.x * cv.zw | (r.y << 16);
+    }
+    for (uint32_t r = threadIdx.x; r <= cv.mb; r += blockDim.x) S.rp[r] = cv.row_ptr[r];
+    return S;
+}
+
+// A workgroup's place in the frame: group, wave and lane, and its scratch rows.
+__device__ __forceinline__ FloodFrame flood_place(const CodeView &cv, const FloodPlan &pl, const FloodLds &S,
+                                                  uint3 *state, float *bel) {
+    const uint32_t kb = cv.nb - cv.mb, w = uni(threadIdx.x >> 6), nw = blockDim.x / 64u / kFloodGroups;
+    const uint32_t g = w / nw, wave = w - g * nw, i = wave * 64u + (threadIdx.x & 63u);
+    return FloodFrame{cv, pl, S, nullptr, state, bel, bel + (size_t)kb * cv.z, g, threadIdx.x & 63u, wave,
+                      min(i, cv.z - 1u), nw, kb, i < cv.z, __builtin_amdgcn_ballot_w64(i < cv.z)};
+}
+
 // EXTRA: some information columns do not fit the LDS.
 template <int ND, bool EXTRA>
 __global__ void __launch_bounds__(kFloodThreads) flood_kernel(FloodArgs a) {
     extern __shared__ __align__(16) uint64_t smem[];
     __shared__ uint32_t s_f, s_done, s_bad[kFloodThreads / 64];
     const CodeView &cv = a.cv;
-    FloodLds S;
-    S.acc = (lds_float *)smem;  // first: its address folds into the offsets of the accesses
-    S.hb = (lds_u64 *)(S.acc + ((a.plan.X * cv.z + 1u) & ~1u));
-    S.carry = (lds_float *)(S.hb + cv.nb * cv.zw);
-    S.chk = (lds_u32 *)(S.carry + 4u * (blockDim.x / kFloodGroups));
-    S.rp = S.chk + cv.nbe;
-    S.done = (lds_u32 *)&s_done;
-    S.bad = (lds_u32 *)s_bad;
-    for (uint32_t e = threadIdx.x; e < cv.nbe; e += blockDim.x) {
-        const uint2 r = cv.row_edge[e];
-        S.chk[e] = r.x * cv.zw | (r.y << 16);
-    }
-    for (uint32_t r = threadIdx.x; r <= cv.mb; r += blockDim.x) S.rp[r] = cv.row_ptr[r];
-    const uint32_t kb = cv.nb - cv.mb, kw = (cv.k + 63) / 64, w = uni(threadIdx.x >> 6);
-    const uint32_t nw = blockDim.x / 64u / kFloodGroups, g = w / nw, wave = w - g * nw;
-    const uint32_t i = wave * 64u + (threadIdx.x & 63u);
-    FloodFrame F{cv, a.plan, S, nullptr, reinterpret_cast<uint3 *>(a.state) + (size_t)blockIdx.x * cv.m,
-                 a.bel + (size_t)blockIdx.x * (cv.n + (size_t)kb * cv.z), nullptr, g, threadIdx.x & 63u, wave,
-                 min(i, cv.z - 1u), nw, kb, i < cv.z, __builtin_amdgcn_ballot_w64(i < cv.z)};
-    F.par = F.info + (size_t)kb * cv.z;
+    const FloodLds S = flood_lds(cv, a.plan, smem, &s_done, s_bad);
+    FloodFrame F = flood_place(cv, a.plan, S, reinterpret_cast<uint3 *>(a.state) + (size_t)blockIdx.x * cv.m,
+                               a.bel + (size_t)blockIdx.x * (cv.n + (size_t)(cv.nb - cv.mb) * cv.z));
+    const uint32_t kw = (cv.k + 63) / 64;
     for (;;) {
         __syncthreads();  // the previous frame is done with the LDS
         if (threadIdx.x == 0) s_f = atomicAdd(a.ctr, 1u);
@@ -478,18 +504,77 @@ __global__ void __launch_bounds__(kFloodThreads) flood_kernel(FloodArgs a) {
     }
 }
 
+// Value of a uniform struct in memory that no running kernel writes, through
+// scalar loads.
+template <typename T>
+__device__ __forceinline__ T ld_uniform(const T *p) {
+    static_assert(sizeof(T) % 4 == 0, "read by words");
+    uint32_t w[sizeof(T) / 4];
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(T) / 4; ++k) w[k] = uni(ldc(reinterpret_cast<const uint32_t *>(p) + k));
+    T v;
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
+}
+
+// Frames of several codes in one launch: each workgroup draws the next frame
+// (the longest codes come first) and runs its code's instantiation.  The
+// registers are those of the largest instantiation, which costs nothing: three
+// waves per SIMD are also what the LDS of a long code allows.  One launch,
+// because a launch per code leaves each with fewer frames than compute units.
+// 2000 frames of the twelve Z=360 codes: 9.6 ms, against 22.8 ms for the
+// iteration graph of the general kernels.
+__global__ void __launch_bounds__(kFloodThreads) flood_mix_kernel(FloodMixArgs a) {
+    extern __shared__ __align__(16) uint64_t smem[];
+    __shared__ uint32_t s_f, s_done, s_bad[kFloodThreads / 64];
+    uint3 *state = reinterpret_cast<uint3 *>(a.state) + (size_t)blockIdx.x * a.state_stride;
+    float *bel = a.bel + (size_t)blockIdx.x * a.bel_stride;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) s_f = atomicAdd(a.ctr, 1u);
+        __syncthreads();
+        const uint32_t j = uni(s_f);
+        if (j >= a.frames) break;
+        const SlotInfo si = ld_uniform(a.jobs + j);
+        const FloodCode fc = ld_uniform(a.codes + si.code);
+        const FloodLds S = flood_lds(fc.cv, fc.plan, smem, &s_done, s_bad);
+        FloodFrame F = flood_place(fc.cv, fc.plan, S, state, bel);
+        F.llr = a.llr + si.llr;
+        bool conv = false;
+        uint32_t its = ~0u;
+        const bool extra = fc.plan.X < fc.cv.nb - fc.cv.mb;
+#define GF2L_FLOOD(ND)                                                                            \
+    case ND:                                                                                      \
+        its = extra ? flood_frame<ND, true>(F, a.max_it, conv) : flood_frame<ND, false>(F, a.max_it, conv); \
+        break;
+        switch (fc.plan.nd) {
+            GF2L_FLOOD_DEGREES
+            default: break;
+        }
+#undef GF2L_FLOOD
+        if (its == ~0u) {
+            if (threadIdx.x == 0) atomicAdd(a.count, 1u);
+            continue;
+        }
+        frame_message(fc.cv, (const uint64_t *)S.hb, a.msg + si.msg);
+        if (threadIdx.x == 0) {
+            a.iters[si.frame] = its;
+            a.conv[si.frame] = (uint8_t)conv;
+            a.synd[si.frame] = (uint8_t)conv;
+        }
+    }
+}
+
 __global__ void clear_words_kernel(uint32_t *p, uint32_t n) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
 // LDS bytes besides the accumulators.
 size_t flood_fixed_bytes(const CodeView &cv, uint32_t lanes) {
-    return (size_t)cv.nb * cv.zw * 8 + 4ull * lanes * sizeof(float) + (size_t)cv.nbe * 4 + (cv.mb + 1ull) * 4 + 4;
+    return (size_t)cv.nb * cv.zw * 8 + 5ull * lanes * sizeof(float) + (size_t)cv.nbe * 4 + (cv.mb + 1ull) * 4 + 4;
 }
 
 uint32_t flood_lanes(uint32_t z) { return (z + 63u) & ~63u; }
-
-constexpr int kFloodDegrees[] = {4, 5, 6, 8, 9, 10, 11, 13, 15, 17, 21, 25};
 
 }  // namespace
 
@@ -519,8 +604,9 @@ int build_flood_plan(gf2l_ctx *ctx, gf2l_code *c) {
         most = std::max(most, d - np);
     }
     uint32_t nd = 0;
-    for (int k : kFloodDegrees)
-        if (!nd && (uint32_t)k >= most) nd = (uint32_t)k;
+#define GF2L_FLOOD(ND) nd = !nd && ND >= most ? ND : nd;
+    GF2L_FLOOD_DEGREES
+#undef GF2L_FLOOD
     const size_t fixed = flood_fixed_bytes(cv, flood_lanes(cv.z)) + 256;
     if (!nd || fixed >= ctx->lds_limit) return GF2L_OK;
     const uint32_t X = (uint32_t)std::min<size_t>(kb, (ctx->lds_limit - fixed) / (cv.z * sizeof(float)));
@@ -571,16 +657,28 @@ int build_flood_plan(gf2l_ctx *ctx, gf2l_code *c) {
     return GF2L_OK;
 }
 
+// Workgroups of a launch: the registers allow three or four waves per SIMD.
 uint32_t flood_grid(const CodeView &cv, const FloodPlan &pl, uint32_t frames, int num_cus) {
     const uint32_t waves = flood_lanes(cv.z) / 64u * kFloodGroups;
     const uint32_t per_cu = (uint32_t)std::max<size_t>(
-        1, std::min<size_t>(32u / waves, (160 * 1024) / (flood_bytes(cv, pl) + 256)));
+        1, std::min<size_t>(12u / waves, (160 * 1024) / (flood_bytes(cv, pl) + 256)));
     return std::max(1u, std::min(frames, (uint32_t)num_cus * per_cu));
 }
 
+hipError_t launch_flood_mix(const FloodMixArgs &a, size_t lds, uint32_t block, uint32_t grid, hipStream_t s) {
+    auto k = flood_mix_kernel;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, s, a);
+    return hipGetLastError();
+}
+
+uint32_t flood_block(const CodeView &cv) { return flood_lanes(cv.z) * kFloodGroups; }
+
 hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s) {
     const size_t bytes = flood_bytes(a.cv, a.plan);
-    const uint32_t block = flood_lanes(a.cv.z) * kFloodGroups;
+    const uint32_t block = flood_block(a.cv);
 #define GF2L_FLOOD(ND)                                                                                       \
     case ND: {                                                                                               \
         auto k = a.plan.X < a.cv.nb - a.cv.mb ? flood_kernel<ND, true> : flood_kernel<ND, false>;            \
@@ -591,8 +689,7 @@ hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s) {
         break;                                                                                               \
     }
     switch (a.plan.nd) {
-        GF2L_FLOOD(4) GF2L_FLOOD(5) GF2L_FLOOD(6) GF2L_FLOOD(8) GF2L_FLOOD(9) GF2L_FLOOD(10)
-        GF2L_FLOOD(11) GF2L_FLOOD(13) GF2L_FLOOD(15) GF2L_FLOOD(17) GF2L_FLOOD(21) GF2L_FLOOD(25)
+        GF2L_FLOOD_DEGREES
         default: return hipErrorInvalidValue;
     }
 #undef GF2L_FLOOD

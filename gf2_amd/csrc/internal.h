@@ -188,6 +188,31 @@ struct FloodArgs {
     uint8_t *conv, *synd;
 };
 
+// Caller-side position of a frame of a mixed-code batch.
+struct SlotInfo {
+    uint32_t frame, code;
+    uint64_t llr, msg;  // element offsets in the caller's packed arrays
+};
+
+// Arguments of the whole-frame kernel over frames of several codes.
+struct FloodCode {
+    CodeView cv;
+    FloodPlan plan;
+};
+struct FloodMixArgs {
+    const FloodCode *codes;
+    const SlotInfo *jobs;    // [frames]
+    const float *llr;
+    uint32_t frames, max_it;
+    uint32_t *state;         // per workgroup state_stride check states (3 words each)
+    float *bel;              // per workgroup bel_stride beliefs
+    uint64_t state_stride, bel_stride;
+    uint32_t *ctr, *count;   // next frame; frames it cannot decode (zeroed before the launch)
+    uint64_t *msg;
+    uint32_t *iters;
+    uint8_t *conv, *synd;
+};
+
 // Arguments of the layered backward kernel (layered.hip).
 struct LayeredBwdArgs {
     CodeView cv;
@@ -361,6 +386,8 @@ size_t flood_bytes(const CodeView &cv, const FloodPlan &pl);
 hipError_t launch_clear_words(uint32_t *words, uint32_t count, hipStream_t s);
 uint32_t flood_grid(const CodeView &cv, const FloodPlan &pl, uint32_t frames, int num_cus);
 hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s);
+uint32_t flood_block(const CodeView &cv);  // threads of its workgroup
+hipError_t launch_flood_mix(const FloodMixArgs &a, size_t lds, uint32_t block, uint32_t grid, hipStream_t s);
 
 // Plain min-sum on a general sparse code (csr.hip).
 int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,

@@ -6,6 +6,7 @@ import pytest
 
 from gf2_amd import _lib, codes
 from gf2_amd.ldpc import Context, LdpcCode, QuasiCyclicLdpc, decode_batch_arrays, qc_ira_base_matrix
+from gf2_amd.mixed import CodeSet, decode_mixed_arrays
 from oracle import oracle as orc
 from tests import frames
 
@@ -59,6 +60,38 @@ def test_matches_oracle(ctx, shape):
         print("[gpu-case] frame kernel", shape, count, max_it, flush=True)
         same(decode(ctx, code, llr[:count], max_it, 2), oc.decode_batch(llr[:count], max_it, threads=8),
              f"{shape} {count}x{max_it}")
+
+
+@pytest.mark.parametrize("special", [False, True])
+def test_mixed_codes(ctx, special):
+    """Frames of codes of different length, row degree and LDS split in one
+    call; with a NaN and an infinite LLR the call is left to the general
+    kernels."""
+    shapes = [(25, 45, 360, [8] * 5 + [3] * 15), (8, 45, 360, [8] + [3] * 36), (5, 120, 360, [1] * 115),
+              (12, 30, 330, [5] * 18)]
+    bases = [qc_ira_base_matrix(7 + i, mb, nb, z, w) for i, (mb, nb, z, w) in enumerate(shapes)]
+    gcodes = [LdpcCode(QuasiCyclicLdpc(b, s[2]), ctx) for b, s in zip(bases, shapes)]
+    ids = np.random.default_rng(2).permutation(np.arange(22) % 4).astype(np.uint16)
+    rows = [frames.random_frames(bases[c], shapes[c][2], 1, (2.6, 3.3, 6.0, 3.0)[c], seed=50 + f)[2][0]
+            for f, c in enumerate(ids)]
+    if special:
+        rows[3][5], rows[9][100:103] = np.nan, np.inf
+    cs = CodeSet(gcodes)
+    out = {}
+    for mode in (1, 2):
+        print("[gpu-case] frame kernel, mixed codes", special, mode, flush=True)
+        ctx.set_tuning(_lib.TUNE_FRAME_KERNEL, mode)
+        try:
+            out[mode] = decode_mixed_arrays(cs, ids, np.concatenate(rows), 30)
+        finally:
+            ctx.set_tuning(_lib.TUNE_FRAME_KERNEL, 0)
+    for a, b in zip(out[1], out[2]):
+        assert np.array_equal(a, b)
+    msg, off, it, conv, synd, _ = out[2]
+    for f, c in enumerate(ids):
+        if np.isfinite(rows[f]).all():
+            ref = orc.Code.from_qc(bases[c], shapes[c][2]).decode_batch(rows[f][None], 30)
+            same([msg[off[f]:off[f + 1]][None], it[f:f + 1], conv[f:f + 1], synd[f:f + 1]], ref, f"frame {f}")
 
 
 def test_more_frames_than_workgroups(ctx):
