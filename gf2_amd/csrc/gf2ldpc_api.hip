@@ -119,6 +119,14 @@ static bool use_frame_kernel(const gf2l_ctx *ctx, const gf2l_code *code, uint32_
     return F >= (code->flood.X == cv.nb - cv.mb ? cus / 6 : cus * 3 / 4);
 }
 
+// Whether a plain batch on the LDS path runs the small codes' whole-frame
+// kernel (faster at every batch size measured, 1 to 16384 frames: 2.0x to 2.7x
+// at N = 2304): unless the path, the thread groups or the kernel was chosen.
+static bool use_small_kernel(const gf2l_ctx *ctx, const gf2l_code *code) {
+    if (!code->small_threads || ctx->tune.frame_kernel == 1) return false;
+    return ctx->tune.frame_kernel == 2 || (ctx->path == gf2l::kAuto && !ctx->tune.lds_groups);
+}
+
 // Plain min-sum by the whole-frame kernel (flood.hip): results of every frame
 // but those in `left` (an LLR or belief too large for it).
 static int decode_flood(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
@@ -214,6 +222,11 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         path = gf2l::kStream;
     }
     if (path < 0) return fail(ctx, GF2L_ERR_UNSUPPORTED, "the forced decoder path cannot run this code");
+    if (path == gf2l::kLds && !d_w && !d_fb && !h_trace_c2v && use_small_kernel(ctx, code)) {
+        GF2L_HIP(ctx, launch_small(cv, code->small_threads, d_llr, F, max_it, d_msg, d_iters, d_conv, d_synd,
+                                   ctx->d_small, ctx->num_cus, s));
+        return GF2L_OK;
+    }
     if (path == gf2l::kLds) {
         float *d_tc = nullptr, *d_tb = nullptr;
         if (h_trace_c2v && trace_iters) {
@@ -617,6 +630,14 @@ int gf2l_create(int device, gf2l_ctx **out) {
             delete ctx;
             return GF2L_ERR_HIP;
         }
+        // here and not on the first decode, which a caller may be recording
+        if (hipMalloc(&ctx->d_small, 2 * sizeof(uint32_t)) != hipSuccess ||
+            hipMemset(ctx->d_small, 0, 2 * sizeof(uint32_t)) != hipSuccess) {
+            hipFree(ctx->d_small);
+            hipStreamDestroy(ctx->stream);
+            delete ctx;
+            return GF2L_ERR_HIP;
+        }
         int cus = 0, lds = 0;
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
         hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
@@ -638,6 +659,7 @@ void gf2l_destroy(gf2l_ctx *ctx) {
     for (auto &e : ctx->prof.lev)
         if (e) hipEventDestroy(e);
     hipFree(ctx->d_io);
+    hipFree(ctx->d_small);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -909,6 +931,7 @@ int gf2l_code_qc(gf2l_ctx *ctx, uint32_t mb, uint32_t nb, uint32_t z, const int3
         }
         int rc = gf2l::build_qc_view(ctx, c, mb, nb, z, 0);
         if (rc != GF2L_OK) return rc;
+        c->small_threads = gf2l::small_threads(c);
         rc = gf2l::build_flood_plan(ctx, c);
         if (rc != GF2L_OK) {
             gf2l_code_destroy(c);

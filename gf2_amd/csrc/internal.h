@@ -242,6 +242,7 @@ struct gf2l_code {
     void *d_tables = nullptr;    // one allocation backing the view's tables
     gf2l::FloodPlan flood;       // whole-frame flooding kernel (d_flood backs its tables)
     void *d_flood = nullptr;
+    uint32_t small_threads = 0;  // workgroup of the small codes' whole-frame kernel (0: not for this code)
     int device = 0;
 };
 
@@ -258,6 +259,7 @@ struct gf2l_ctx {
     size_t lds_limit = 0;        // bytes of dynamic LDS one workgroup may use
     std::string err;
     gf2l::Workspace ws;
+    uint32_t *d_small = nullptr; // frame counters of the small codes' kernel (zero between launches)
     // staging for the host-pointer entry point
     void *d_io = nullptr;
     size_t d_io_bytes = 0;
@@ -388,6 +390,14 @@ uint32_t flood_grid(const CodeView &cv, const FloodPlan &pl, uint32_t frames, in
 hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s);
 uint32_t flood_block(const CodeView &cv);  // threads of its workgroup
 hipError_t launch_flood_mix(const FloodMixArgs &a, size_t lds, uint32_t block, uint32_t grid, hipStream_t s);
+
+// Whole-frame kernel of small codes on the LDS path (small.hip): its workgroup
+// for a code (0: the code does not suit it) and the launcher.  ctr: two words,
+// zero before the first launch and left at zero (null: a fixed stride).
+uint32_t small_threads(const gf2l_code *code);
+hipError_t launch_small(const CodeView &cv, uint32_t threads, const float *llr, uint32_t frames, uint32_t max_it,
+                        uint64_t *msg, uint32_t *iters, uint8_t *conv, uint8_t *synd, uint32_t *ctr, int num_cus,
+                        hipStream_t s);
 
 // Plain min-sum on a general sparse code (csr.hip).
 int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,

@@ -184,10 +184,12 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
  *                        profiling or tracing, never by the no-allocation
  *                        entry point.
  *   GF2L_TUNE_FRAME_KERNEL plain decodes of staircase quasi-cyclic codes on
- *                        the STATE path: 0 (default) one workgroup per frame
+ *                        the STATE path, and of codes of check degree 2 to 8 on
+ *                        the LDS path: 0 (default) one workgroup per frame
  *                        for all its iterations where that is faster (never
- *                        on a forced path), 1 never, 2 wherever the code has
- *                        the structure. */
+ *                        on a forced path, nor with GF2L_TUNE_LDS_GROUPS or
+ *                        GF2L_TUNE_HBM_GRAPH set), 1 never (LDS path: its
+ *                        general kernel), 2 wherever the code allows it. */
 #define GF2L_TUNE_WG_PER_CU 1
 #define GF2L_TUNE_XCD_MAP 2
 #define GF2L_TUNE_GRAPH_ITERS 3

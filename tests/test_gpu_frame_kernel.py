@@ -62,6 +62,59 @@ def test_matches_oracle(ctx, shape):
              f"{shape} {count}x{max_it}")
 
 
+def random_base(mb, nb, z, degree, seed):
+    """Any base matrix: rows of up to `degree` circulants, no structure."""
+    rng = np.random.default_rng(seed)
+    base = -np.ones((mb, nb), dtype=np.int32)
+    for r in range(mb):
+        cols = rng.choice(nb, size=int(rng.integers(2, degree + 1)), replace=False)
+        base[r, cols] = rng.integers(0, z, size=cols.size)
+    return base
+
+
+# (mb, nb, z, largest row degree): one check, checks and variables that fill
+# no wave, a whole wave, both degree classes, columns without a check, the
+# largest workgroups
+SMALL = {"one-check": (1, 3, 1, 3), "under-a-wave": (4, 9, 7, 6), "one-wave": (3, 6, 64, 5),
+         "degree-8": (9, 18, 65, 8), "many-columns": (6, 40, 50, 8), "n2304": (12, 24, 96, 6),
+         "ten-waves": (16, 32, 120, 6), "fourteen-waves": (26, 52, 100, 3)}
+
+
+@pytest.mark.parametrize("shape", SMALL)
+def test_small_codes_match_oracle(ctx, shape):
+    mb, nb, z, degree = SMALL[shape]
+    base = random_base(mb, nb, z, degree, 21)
+    code = LdpcCode(QuasiCyclicLdpc(base, z), ctx)
+    assert ctx.code_path(code) == _lib.PATH_LDS
+    oc = orc.Code.from_qc(base, z)
+    rng = np.random.default_rng(22)
+    llr = rng.normal(1.0, 1.4, size=(41, nb * z)).astype(np.float32)  # the zero codeword, noisy
+    llr[rng.random(llr.shape) < 0.01] = -0.0
+    llr[rng.random(llr.shape) < 0.01] = 0.0
+    for count, max_it in ((1, 30), (41, 1), (41, 30)):
+        print("[gpu-case] small-code kernel", shape, count, max_it, flush=True)
+        same(decode(ctx, code, llr[:count], max_it, 0), oc.decode_batch(llr[:count], max_it, threads=8),
+             f"{shape} {count}x{max_it}")
+
+
+def test_small_codes_many_frames_and_special_llrs(ctx):
+    """More frames than workgroups, twice (the frame counter starts over), with
+    infinite, NaN and very large LLRs in some frames: as the general kernel."""
+    spec = codes.n2304_r12()
+    base = spec.base_matrix()
+    code = LdpcCode(QuasiCyclicLdpc(base, spec.z), ctx)
+    _, _, llr = frames.random_frames(base, spec.z, 300, 2.0, seed=6)
+    rng = np.random.default_rng(7)
+    for f, v in ((1, np.inf), (4, -np.inf), (7, np.nan), (9, 2e30), (10, -3.3e38), (12, -np.nan)):
+        llr[f, rng.integers(0, spec.n, 9)] = v
+    llr[11] *= np.float32(1e28)  # beliefs pass the limit while it iterates
+    llr = np.tile(llr, (9, 1))
+    print("[gpu-case] small-code kernel, 2700 frames", flush=True)
+    ref = decode(ctx, code, llr, 50, 1)
+    for _ in range(2):
+        same(decode(ctx, code, llr, 50, 0), ref, "small")
+
+
 @pytest.mark.parametrize("special", [False, True])
 def test_mixed_codes(ctx, special):
     """Frames of codes of different length, row degree and LDS split in one
