@@ -160,7 +160,7 @@ struct LayeredArgs {
     uint32_t X;              // block-columns whose beliefs live in LDS (0..X-1)
     int fallback;            // frames failing after T: 1 -> continuation list, 0 -> retire
     uint32_t *state;         // [F][mb][zp][3] compressed check states
-    const uint3 *zero_state; // staircase kernel: [mb][zp] zero states, read in place of iteration 1's
+    const uint3 *zero_state; // staircase kernel: [mb][zp] zero states (16 bytes each), read in place of iteration 1's
     float *belief;           // [F][nb][zp] beliefs of block-columns >= X (all at hand-over)
     uint32_t *ctr;           // [0] next frame, [1] layered frame-iterations run (zeroed by the host)
     uint32_t *list, *count;  // running list of the continuation and its length
@@ -227,6 +227,7 @@ struct LayeredBwdArgs {
     float scale;              // 1 / (T n F)
     float *lpart;             // [F] loss of each frame
     uint32_t *ctr;            // [0] next frame (zeroed by the host)
+    uint64_t stair_deg[4], stair_sync[4];  // staircase kernel: as in LayeredArgs
 };
 
 }  // namespace gf2l
@@ -378,7 +379,9 @@ hipError_t launch_layered_bwd(const LayeredBwdArgs &a, int num_cus, hipStream_t 
 // LayeredArgs::stair_deg and stair_sync) and its launcher.
 size_t layered_stair_bytes(const CodeView &cv);
 uint32_t layered_stair_degree(const gf2l_code *code, uint64_t *deg_mask = nullptr, uint64_t *sync_mask = nullptr);
-hipError_t launch_layered_stair(const LayeredArgs &a, uint32_t dh, int num_cus, hipStream_t s);
+hipError_t launch_layered_stair(const LayeredArgs &a, uint32_t dh, bool tape, int num_cus, hipStream_t s);
+size_t layered_stair_bwd_bytes(const CodeView &cv);
+hipError_t launch_layered_stair_bwd(const LayeredBwdArgs &a, uint32_t dh, int num_cus, hipStream_t s);
 
 // Whole-frame flooding kernel (flood.hip): builds the row tables of a
 // quasi-cyclic code that has the structure (leaves code->flood empty

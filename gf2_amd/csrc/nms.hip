@@ -33,7 +33,7 @@ struct gf2l_nms {
     bool fb_continue = false; // the plain fallback continues from the learned state (layered: always)
     uint32_t X = 0;           // layered: block-columns whose beliefs a workgroup keeps in LDS
     float *d_w = nullptr;     // [T][nbe]
-    uint32_t *d_zero_state = nullptr;  // layered: [mb][zp][3] zeros, iteration 1's check states
+    uint32_t *d_zero_state = nullptr;  // layered: [mb][zp][4] zeros, iteration 1's check states
     float *d_m = nullptr;     // Adam first moment
     float *d_v = nullptr;     // Adam second moment
     uint64_t step = 0;
@@ -307,7 +307,7 @@ int ensure_train(gf2l_ctx *ctx, gf2l_nms *q, size_t F) {
     const size_t rec = q->layered ? 4 : 3;  // words per tape record of a check
     GF2L_HIP(ctx, hipMalloc(&q->tape_state, T * F * rec * cv.mb * cv.zp * sizeof(uint32_t)));
     GF2L_HIP(ctx, hipMalloc(&q->tape_bel, T * F * cv.nb * cv.zp * sizeof(float)));
-    GF2L_HIP(ctx, hipMalloc(&q->g_a, F * E * sizeof(float)));
+    GF2L_HIP(ctx, hipMalloc(&q->g_a, F * (E + cv.z) * sizeof(float)));  // layered: a row past a frame's last edge is read
     if (!q->layered) GF2L_HIP(ctx, hipMalloc(&q->g_b, F * E * sizeof(float)));
     GF2L_HIP(ctx, hipMalloc(&q->g_bel, F * cv.nb * cv.zp * sizeof(float)));
     GF2L_HIP(ctx, hipMalloc(&q->gpart, T * cv.nbe * F * sizeof(float)));
@@ -378,13 +378,21 @@ int layered_forward_backward(gf2l_ctx *ctx, gf2l_nms *q, const float *d_llr, con
     a.count = q->count + 3;
     a.tape_state = q->tape_state;
     a.tape_bel = q->tape_bel;
-    GF2L_HIP(ctx, launch_layered_fwd(a, true, ctx->num_cus, s));
+    const int dh = layered_stair(ctx, q);
+    if (dh > 0) {
+        a.X = cv.nb - cv.mb;
+        a.zero_state = reinterpret_cast<const uint3 *>(q->d_zero_state);
+        layered_stair_degree(q->code, a.stair_deg, a.stair_sync);
+        GF2L_HIP(ctx, launch_layered_stair(a, (uint32_t)dh, true, ctx->num_cus, s));
+    } else {
+        GF2L_HIP(ctx, launch_layered_fwd(a, true, ctx->num_cus, s));
+    }
     LayeredBwdArgs b{};
     b.cv = cv;
     b.w = q->d_w;
     b.F = F;
     b.T = T;
-    b.X = a.X;
+    b.X = layered_x(ctx, q);
     b.tape_state = q->tape_state;
     b.tape_bel = q->tape_bel;
     b.cw = d_cw;
@@ -394,7 +402,12 @@ int layered_forward_backward(gf2l_ctx *ctx, gf2l_nms *q, const float *d_llr, con
     b.scale = 1.0f / ((float)T * (float)cv.n * (float)F);
     b.lpart = q->lpart;
     b.ctr = q->count + 2;
-    GF2L_HIP(ctx, launch_layered_bwd(b, ctx->num_cus, s));
+    if (dh > 0 && layered_stair_bwd_bytes(cv) + 128 <= ctx->lds_limit) {
+        layered_stair_degree(q->code, b.stair_deg, b.stair_sync);
+        GF2L_HIP(ctx, launch_layered_stair_bwd(b, (uint32_t)dh, ctx->num_cus, s));
+    } else {
+        GF2L_HIP(ctx, launch_layered_bwd(b, ctx->num_cus, s));
+    }
     hipLaunchKernelGGL(grad_reduce_kernel, dim3(T * cv.nbe), dim3(256), 0, s, q->gpart, F, q->grad);
     hipLaunchKernelGGL(grad_reduce_kernel, dim3(1), dim3(256), 0, s, q->lpart, F, q->loss);
     GF2L_HIP(ctx, hipGetLastError());
@@ -441,7 +454,7 @@ int layered_decode(gf2l_ctx *ctx, const gf2l_nms *q, const float *d_llr, uint32_
     a.fb = d_fb;
     if (pf.on) GF2L_HIP(ctx, hipEventRecord(pf.lev[0], s));
     if (dh > 0)
-        GF2L_HIP(ctx, launch_layered_stair(a, (uint32_t)dh, ctx->num_cus, s));
+        GF2L_HIP(ctx, launch_layered_stair(a, (uint32_t)dh, false, ctx->num_cus, s));
     else
         GF2L_HIP(ctx, launch_layered_fwd(a, false, ctx->num_cus, s));
     if (pf.on) GF2L_HIP(ctx, hipEventRecord(pf.lev[1], s));
@@ -595,7 +608,7 @@ int create_nms(gf2l_ctx *ctx, const gf2l_code *code, uint32_t iterations, const 
     if (e == hipSuccess) e = hipMemcpy(q->d_w, w.data(), nw * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(q->d_m, 0, nw * sizeof(float));
     if (e == hipSuccess) e = hipMemset(q->d_v, 0, nw * sizeof(float));
-    const size_t zbytes = 3ull * code->view.mb * code->view.zp * sizeof(uint32_t);
+    const size_t zbytes = 4ull * code->view.mb * code->view.zp * sizeof(uint32_t);
     if (e == hipSuccess && layered) e = hipMalloc(&q->d_zero_state, zbytes);
     if (e == hipSuccess && layered) e = hipMemset(q->d_zero_state, 0, zbytes);
     if (e != hipSuccess) {
