@@ -189,7 +189,9 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
  *                        for all its iterations where that is faster (never
  *                        on a forced path, nor with GF2L_TUNE_LDS_GROUPS or
  *                        GF2L_TUNE_HBM_GRAPH set), 1 never (LDS path: its
- *                        general kernel), 2 wherever the code allows it. */
+ *                        general kernel), 2 wherever the code allows it.
+ *                        General sparse codes: 1 keeps each frame's arrays
+ *                        contiguous instead of 64 frames interleaved. */
 #define GF2L_TUNE_WG_PER_CU 1
 #define GF2L_TUNE_XCD_MAP 2
 #define GF2L_TUNE_GRAPH_ITERS 3
