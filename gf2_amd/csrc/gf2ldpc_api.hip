@@ -127,6 +127,27 @@ static bool use_small_kernel(const gf2l_ctx *ctx, const gf2l_code *code) {
     return ctx->tune.frame_kernel == 2 || (ctx->path == gf2l::kAuto && !ctx->tune.lds_groups);
 }
 
+// Whether a plain batch runs the team kernel, and its sizes.
+static bool use_team(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F, uint32_t max_it, TeamArgs &a) {
+    const int mode = ctx->tune.frame_kernel;
+    if (mode == 1 || mode == 2 || !team_shape(code->view, F, max_it, ctx->num_cus, ctx->lds_limit, a)) return false;
+    if (mode >= 3) return true;
+    if (ctx->path != gf2l::kAuto || ctx->tune.hbm_graph || ctx->prof.on) return false;
+    // DVB codes: faster than the state kernels at every batch size and rate
+    // (normal r 1/2: 1 frame 1013 -> 245 us, 202 frames 4.23 -> 3.61 ms, 1000
+    // frames 14.8 -> 14.2 ms; r 2/3: 1000 frames 16.1 -> 11.4 ms; short r 1/2:
+    // 1000 frames 5.03 -> 3.42 ms).
+    if (!code->flood.nd) return true;
+    // Codes of the whole-frame kernel.  Those with two of its workgroups to a
+    // compute unit (N = 16200, r 0.44): teams of four or more win (1 frame 255 ->
+    // 137 us, 64 frames 386 -> 306 us), teams of two lose (100 frames 430 -> 541
+    // us).  Longer ones: wherever every frame has a team at once (N = 64800: 24
+    // frames 1446 -> 480 us, 85 frames 2.71 -> 2.42 ms, at r 2/3 128 frames 1.35
+    // -> 1.33 ms; with a second turn 128 frames at r 1/2 2.72 -> 2.92 ms).
+    if (flood_bytes(code->view, code->flood) <= 80 * 1024) return a.team >= 4;
+    return F <= a.teams && a.team > 1;
+}
+
 // Plain min-sum by the whole-frame kernel (flood.hip): results of every frame
 // but those in `left` (an LLR or belief too large for it).
 static int decode_flood(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
@@ -174,6 +195,51 @@ static int decode_flood(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr
         GF2L_HIP(ctx, hipStreamSynchronize(s));
         std::sort(left.begin(), left.end());
     }
+    return GF2L_OK;
+}
+
+// Plain min-sum of a batch, or of the frames `only` of it, by the team kernel
+// (team.hip).  done: false if its workgroups did not all come to run at once
+// (results of these frames are then not to be used).
+static int decode_team(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
+                       TeamArgs &a, const std::vector<uint32_t> *only, uint64_t *d_msg, uint32_t *d_iters,
+                       uint8_t *d_conv, uint8_t *d_synd, bool &done) {
+    const CodeView &cv = code->view;
+    hipStream_t s = ctx->stream;
+    const size_t sync = (size_t)a.teams * kTeamSyncStride;
+    int rc = ensure_buffers(ctx, F, a.team > 1 ? (size_t)cv.nbe * cv.zp * a.teams : 0, 0,
+                            (size_t)cv.nb * cv.zp * a.teams, sync,
+                            a.llr_words);
+    if (rc != GF2L_OK) return rc;
+    Workspace &ws = ctx->ws;
+    GF2L_HIP(ctx, launch_clear_words(reinterpret_cast<uint32_t *>(ws.hb), (uint32_t)(2 * sync), s));
+    GF2L_HIP(ctx, launch_clear_words(ws.counts, 2, s));
+    a.cv = cv;
+    a.llr = d_llr;
+    a.frames = only ? (uint32_t)only->size() : F;
+    if (only) {
+        GF2L_HIP(ctx, hipMemcpyAsync(ws.lists, only->data(), only->size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+        a.list = ws.lists;
+    }
+    a.max_it = max_it;
+    a.llr_own = ws.llr_perm;
+    a.msg = ws.c2v;
+    a.bel = ws.belief;
+    a.sync = ws.hb;
+    a.gave_up = ws.counts;
+    a.queue = ws.counts + 1;
+    // a team whose workgroups are not all there after 300 us is waiting for
+    // other work on the chip; once they are, a wait is as long as one pass
+    a.first_wait = ctx->tune.frame_kernel == 4 ? 0u : 30000u;
+    a.wait = 20000000u;
+    a.msg_out = d_msg;
+    a.iters = d_iters;
+    a.conv = d_conv;
+    a.synd = d_synd;
+    GF2L_HIP(ctx, launch_team(a, s));
+    GF2L_HIP(ctx, hipMemcpyAsync(ws.h_count, ws.counts, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    GF2L_HIP(ctx, hipStreamSynchronize(s));
+    done = ws.h_count[0] == 0;
     return GF2L_OK;
 }
 
@@ -246,6 +312,36 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
             hipFree(d_tb);
         }
         return GF2L_OK;
+    }
+    if (path == gf2l::kState && !d_w && !d_fb && !h_trace_c2v) {
+        TeamArgs team{};
+        bool done = false;
+        if (use_team(ctx, code, F, max_it, team)) {
+            std::vector<uint32_t> rest;
+            const bool first = team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3;
+            if (first) {
+                // Teams take several frames each: the first iteration by the
+                // state kernels, which are faster at it (202 error-free frames
+                // of DVB-T2 normal r 3/5: 292 us with the iterations they queue
+                // behind it, 345 by teams; in noise the teams alone would take
+                // 3% to 16% less), then teams for the frames still running.
+                int rc1 = ensure_workspace(ctx, cv, path, F);
+                if (rc1 == GF2L_OK)
+                    rc1 = run_hbm(ctx, cv, path, ctx->ws, d_llr, F, 1, nullptr, 0, false, d_msg, d_iters, d_conv, d_synd,
+                                  nullptr, nullptr, nullptr, 0, nullptr, nullptr, false, nullptr);
+                if (rc1 != GF2L_OK || max_it == 1) return rc1;
+                std::vector<uint8_t> conv(F);
+                GF2L_HIP(ctx, hipMemcpyAsync(conv.data(), d_conv, F, hipMemcpyDeviceToHost, s));
+                GF2L_HIP(ctx, hipStreamSynchronize(s));
+                for (uint32_t f = 0; f < F; ++f)
+                    if (!conv[f]) rest.push_back(f);
+                if (rest.empty()) return GF2L_OK;
+                use_team(ctx, code, (uint32_t)rest.size(), max_it, team);  // sizes for fewer frames
+            }
+            const int rct = decode_team(ctx, code, d_llr, F, max_it, team, first ? &rest : nullptr, d_msg, d_iters,
+                                        d_conv, d_synd, done);
+            if (rct != GF2L_OK || done) return rct;
+        }
     }
     std::vector<uint32_t> left;  // frames the whole-frame kernel leaves to the general ones
     bool whole = false;
@@ -883,7 +979,7 @@ int gf2l_set_tuning(gf2l_ctx *ctx, int key, int value) {
                 ctx->tune.hbm_graph = value;
                 return GF2L_OK;
             case GF2L_TUNE_FRAME_KERNEL:
-                if (value < 0 || value > 2) return fail(ctx, GF2L_ERR_INVALID, "frame kernel out of [0,2]");
+                if (value < 0 || value > 4) return fail(ctx, GF2L_ERR_INVALID, "frame kernel out of [0,4]");
                 ctx->tune.frame_kernel = value;
                 return GF2L_OK;
             case GF2L_TUNE_LDS_GROUPS:

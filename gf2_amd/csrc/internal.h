@@ -117,7 +117,7 @@ struct Tuning {
     int layered_kernel = 0; // 0: staircase kernel where it applies, 1: general kernel, 2: staircase kernel
     int lds_groups = 0;  // thread groups per workgroup of the LDS path (0: automatic)
     int hbm_graph = 0;   // 1: plain iterations of the HBM paths replayed from a captured graph
-    int frame_kernel = 0; // whole-frame flooding kernel: 0 automatic, 1 never, 2 wherever the code allows it
+    int frame_kernel = 0; // one-launch kernels: 0 automatic, 1 never, 2 workgroup per frame, 3 teams, 4 teams that do not wait
 };
 
 // Word offset of the item counters in Workspace::counts and its size (two
@@ -187,6 +187,29 @@ struct FloodArgs {
     uint32_t *iters;
     uint8_t *conv, *synd;
 };
+
+// Arguments of the team kernel (team.hip): small batches, a frame spread over
+// several workgroups.
+struct TeamArgs {
+    CodeView cv;
+    const float *llr;        // [frames][n], the caller's order
+    const uint32_t *list;    // the frames to decode (null: all)
+    uint32_t frames, max_it; // frames: entries of list
+    uint32_t team, teams;    // workgroups per frame, frames at a time (grid: team * teams)
+    uint32_t lds, llr_lds;   // bytes of LDS; whether the channel LLRs are in it
+    size_t llr_words;        // otherwise floats of llr_own
+    float *llr_own;          // per workgroup, by owning thread
+    float *msg;              // per team [nbe][zp] check messages
+    float *bel;              // per team [nb][zp] beliefs
+    uint64_t *sync;          // per team, kTeamSyncStride apart: meeting counter (zeroed before the launch)
+    uint32_t *queue;         // frames taken past the first of each team (zeroed before the launch)
+    uint32_t *gave_up;       // set when a wait ended without the team (zeroed before the launch)
+    uint32_t wait, first_wait;  // longest waits in 10 ns ticks
+    uint64_t *msg_out;
+    uint32_t *iters;
+    uint8_t *conv, *synd;
+};
+constexpr uint32_t kTeamSyncStride = 16;
 
 // Caller-side position of a frame of a mixed-code batch.
 struct SlotInfo {
@@ -393,6 +416,11 @@ uint32_t flood_grid(const CodeView &cv, const FloodPlan &pl, uint32_t frames, in
 hipError_t launch_flood(const FloodArgs &a, uint32_t grid, hipStream_t s);
 uint32_t flood_block(const CodeView &cv);  // threads of its workgroup
 hipError_t launch_flood_mix(const FloodMixArgs &a, size_t lds, uint32_t block, uint32_t grid, hipStream_t s);
+
+// Sizes of the team kernel for `frames` frames of a code (false: it does not
+// suit the code or the batch) and the launcher.
+bool team_shape(const CodeView &cv, uint32_t frames, uint32_t max_it, int num_cus, size_t lds_limit, TeamArgs &a);
+hipError_t launch_team(const TeamArgs &a, hipStream_t s);
 
 // Whole-frame kernel of small codes on the LDS path (small.hip): its workgroup
 // for a code (0: the code does not suit it) and the launcher.  ctr: two words,

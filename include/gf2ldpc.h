@@ -183,15 +183,20 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
  *                        0 (default): launched one by one.  Never while
  *                        profiling or tracing, never by the no-allocation
  *                        entry point.
- *   GF2L_TUNE_FRAME_KERNEL plain decodes of staircase quasi-cyclic codes on
- *                        the STATE path, and of codes of check degree 2 to 8 on
- *                        the LDS path: 0 (default) one workgroup per frame
- *                        for all its iterations where that is faster (never
- *                        on a forced path, nor with GF2L_TUNE_LDS_GROUPS or
- *                        GF2L_TUNE_HBM_GRAPH set), 1 never (LDS path: its
- *                        general kernel), 2 wherever the code allows it.
- *                        General sparse codes: 1 keeps each frame's arrays
- *                        contiguous instead of 64 frames interleaved. */
+ *   GF2L_TUNE_FRAME_KERNEL plain decodes by kernels that run all iterations
+ *                        of a frame in one launch, in place of the general
+ *                        kernels of the STATE path (a workgroup per frame for
+ *                        staircase quasi-cyclic codes; a team of workgroups
+ *                        per frame for small batches and DVB codes), of the
+ *                        LDS path (check degrees 2 to 8) and of general sparse
+ *                        codes (64 frames interleaved): 0 (default) where that
+ *                        is faster (never on a forced path, nor with
+ *                        GF2L_TUNE_LDS_GROUPS or GF2L_TUNE_HBM_GRAPH set; no
+ *                        teams while profiling), 1 never, 2 a workgroup per
+ *                        frame wherever the code allows it, 3 teams wherever
+ *                        the code allows it, 4 as 3, but a team whose
+ *                        workgroups do not meet at once leaves the batch to
+ *                        the general kernels (otherwise after 0.3 ms). */
 #define GF2L_TUNE_WG_PER_CU 1
 #define GF2L_TUNE_XCD_MAP 2
 #define GF2L_TUNE_GRAPH_ITERS 3
