@@ -70,3 +70,21 @@ def test_fer_sweep_any_code(ctx):
     a = fer.sweep(qc, [2.0], 1024, 4096, 10**6, zero_codeword=False)[0]
     b = fer.sweep(qc, [2.0], 1024, 4096, 10**6, zero_codeword=True)[0]
     assert abs(a.fer - b.fer) < 5 * np.sqrt(max(a.fer, 1e-3) / 4096) + 0.01
+
+
+# an odd n (single stores), a lift where n * z passes 2^32 (divisions), the
+# smallest lift
+@pytest.mark.parametrize("mb,nb,z", [(3, 7, 101), (2, 4, 70000), (2, 5, 64)])
+def test_framegen_shapes_match_oracle(ctx, mb, nb, z):
+    from gf2_amd.ldpc import qc_ira_base_matrix
+    base = qc_ira_base_matrix(3, mb, nb, z, [2] * (nb - mb))
+    code = LdpcCode(QuasiCyclicLdpc(base, z), ctx)
+    n, F = nb * z, 3
+    print("[gpu-case] framegen shape", mb, nb, z, flush=True)
+    d_llr, d_cw = generate_frames(code, 99, 7, F, 0.0, 4.0)
+    llr = d_llr.download(np.float32, (F, n))
+    cw = d_cw.download(np.uint64, (F, (n + 63) // 64))
+    for f in range(F):
+        rl, rcw = orc.framegen(base, z, 99, 7 + f, 0.0, 4.0)
+        assert np.array_equal(cw[f], rcw), f
+        np.testing.assert_allclose(llr[f], rl, rtol=2e-6, atol=1e-6)
