@@ -302,22 +302,44 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
         // The strict-comparison update (a < m1: m2 = m1, m1 = a; else a < m2:
         // m2 = a) as min / median: with m1 <= m2 the new m2 is the median of
         // (m1, a, m2) and the new m1 is min(m1, a), the same values for any
-        // non-NaN a (|x| carries no -0); idx keeps the strict comparison, so
-        // the first of equal magnitudes keeps it.
+        // non-NaN a (|x| carries no -0); TAPE: idx keeps the strict
+        // comparison, so the first of equal magnitudes keeps it.
         const float av = fabsf(x[p]);
-        if constexpr (TAPE) idx2 = av < m1 ? idx : (av < m2 ? (uint32_t)p : idx2);
-        idx = av < m1 ? (uint32_t)p : idx;
+        if constexpr (TAPE) {
+            idx2 = av < m1 ? idx : (av < m2 ? (uint32_t)p : idx2);
+            idx = av < m1 ? (uint32_t)p : idx;
+            lt |= (x[p] < 0.0f ? 1u : 0u) << p;
+        }
         m2 = __builtin_amdgcn_fmed3f(m1, av, m2);
         m1 = __builtin_fminf(m1, av);
-        lt |= (x[p] < 0.0f ? 1u : 0u) << p;
     }
-    const uint32_t sg = ((__popc(lt) & 1u) ? (1u << D) - 1u : 0u) ^ lt;  // output sign bits
-    const uint32_t meta = idx | (sg << 5);
+    // Decoding takes the signs as sign bits, shifted in one instruction an
+    // input: a -0.0 input counts as negative then, which turns the sign of
+    // messages of magnitude zero only (its own message does not depend on it),
+    // and no zero's sign reaches a decision, a count or a nonzero belief.
+    if constexpr (!TAPE)
+#pragma unroll
+        for (int p = D - 1; p >= 0; --p) lt = __builtin_amdgcn_alignbit(lt, __float_as_uint(x[p]), 31u);
+    const uint32_t odd = __popc(lt) & 1u;
+    const uint32_t sg = (odd ? (1u << D) - 1u : 0u) ^ lt;  // output sign bits
+    // magnitudes with the parity of all signs; a message's sign is that and
+    // its own input's
+    const uint32_t m1s = __float_as_uint(m1) | (odd << 31), m2s = __float_as_uint(m2) | (odd << 31);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int p = 0; p < D; ++p) {
-        const float mag = (uint32_t)p == idx ? m2 : m1;
-        const float v = x[p] + flip(wt[p] * mag, (sg >> p) & 1u);
+        float v;
+        if constexpr (TAPE) {
+            const float mag = (uint32_t)p == idx ? m2 : m1;
+            v = x[p] + flip(wt[p] * mag, (sg >> p) & 1u);
+        } else {
+            // the input of least magnitude gets m2; where two are equal so are
+            // m1 and m2, and either may keep the place
+            const bool least = fabsf(x[p]) == m1;
+            idx = least ? (uint32_t)p : idx;
+            const uint32_t mag = least ? m2s : m1s;
+            v = x[p] + wt[p] * __uint_as_float(mag ^ (__float_as_uint(x[p]) & 0x80000000u));
+        }
         if (p == D - 1) {
             carry = v;  // column kb+br: to layer br+1, final now for the last block-row
             stu(S.gb + (S.kb + br) * cv.zp, S.i, v);
@@ -342,6 +364,7 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
             lds_st(ad[p], v);
         }
     }
+    const uint32_t meta = idx | (sg << 5);
     if constexpr (TAPE)
         stu(S.tp + br * cv.zp, S.i,
             make_uint4(__float_as_uint(m1), __float_as_uint(m2), meta,
