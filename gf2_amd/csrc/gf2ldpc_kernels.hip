@@ -614,19 +614,45 @@ hipError_t launch_lds_t(const CodeView &cv, LdsShape shp, const float *llr, uint
 }
 
 // LLRs in the standard's bit order -> quasi-cyclic order of a DVB code:
-// parity bit k + a + q*b moves to k + a*z + b (a < q, b < z).
-__global__ void dvb_permute_kernel(CodeView cv, const float *__restrict__ llr, float *__restrict__ out,
-                                   uint32_t frames) {
-    const size_t total = (size_t)frames * cv.n;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-        const size_t f = t / cv.n;
-        const uint32_t u = (uint32_t)(t - f * cv.n);
-        uint32_t v = u;
-        if (u >= cv.k) {
-            const uint32_t w = u - cv.k, a = w / cv.z, b = w - a * cv.z;
-            v = cv.k + a + cv.dvb_q * b;
+// parity bit k + a + q*b moves to k + a*z + b (a < q, b < z).  A workgroup
+// copies a piece of the information part of a frame or transposes a tile of the
+// parity part through LDS, so both sides move whole rows (read element by
+// element with stride q, 202 frames of N = 64800 took 42 us, now 26).
+constexpr uint32_t kPermPiece = 4096, kPermTile = 64;
+__global__ void __launch_bounds__(256)
+dvb_permute_kernel(CodeView cv, const float *__restrict__ llr, float *__restrict__ out, uint32_t frames,
+                   uint32_t pieces, uint32_t tiles_a, uint32_t jobs) {
+    __shared__ float tile[kPermTile][kPermTile + 1];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t total = (uint64_t)frames * jobs;
+    for (uint64_t t = blockIdx.x; t < total; t += gridDim.x) {
+        const uint32_t f = (uint32_t)(t / jobs), job = (uint32_t)(t - (uint64_t)f * jobs);
+        const float *in = llr + (size_t)f * cv.n;
+        float *o = out + (size_t)f * cv.n;
+        if (job < pieces) {
+            const uint32_t u0 = job * kPermPiece + threadIdx.x;
+            float v[kPermPiece / 256];
+#pragma unroll
+            for (uint32_t r = 0; r < kPermPiece / 256; ++r) v[r] = u0 + 256u * r < cv.k ? in[u0 + 256u * r] : 0.0f;
+#pragma unroll
+            for (uint32_t r = 0; r < kPermPiece / 256; ++r)
+                if (u0 + 256u * r < cv.k) o[u0 + 256u * r] = v[r];
+            continue;
         }
-        out[t] = llr[f * cv.n + v];
+        const uint32_t tb = (job - pieces) / tiles_a, ta = job - pieces - tb * tiles_a;
+        const uint32_t a0 = ta * kPermTile, b0 = tb * kPermTile;
+        __syncthreads();  // the previous tile has been written out
+#pragma unroll
+        for (uint32_t r = 0; r < kPermTile / 4; ++r) {
+            const uint32_t b = 4u * r + wave;
+            if (b0 + b < cv.z && a0 + lane < cv.dvb_q) tile[b][lane] = in[cv.k + a0 + lane + cv.dvb_q * (b0 + b)];
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < kPermTile / 4; ++r) {
+            const uint32_t a = 4u * r + wave;
+            if (a0 + a < cv.dvb_q && b0 + lane < cv.z) o[cv.k + (a0 + a) * cv.z + b0 + lane] = tile[lane][a];
+        }
     }
 }
 
@@ -634,9 +660,10 @@ __global__ void dvb_permute_kernel(CodeView cv, const float *__restrict__ llr, f
 
 hipError_t launch_dvb_permute(const CodeView &cv, const float *llr, float *out, uint32_t frames, hipStream_t s) {
     if (frames == 0) return hipSuccess;
-    const size_t total = (size_t)frames * cv.n;
-    const uint32_t grid = (uint32_t)std::min<size_t>((total + 255) / 256, 65536);
-    hipLaunchKernelGGL(dvb_permute_kernel, dim3(grid), dim3(256), 0, s, cv, llr, out, frames);
+    const uint32_t pieces = (cv.k + kPermPiece - 1) / kPermPiece, tiles_a = (cv.dvb_q + kPermTile - 1) / kPermTile;
+    const uint32_t jobs = pieces + tiles_a * ((cv.z + kPermTile - 1) / kPermTile);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)frames * jobs, 65536);
+    hipLaunchKernelGGL(dvb_permute_kernel, dim3(grid), dim3(256), 0, s, cv, llr, out, frames, pieces, tiles_a, jobs);
     return hipGetLastError();
 }
 
