@@ -198,29 +198,34 @@ static int decode_flood(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr
     return GF2L_OK;
 }
 
-// Plain min-sum of a batch, or of the frames `only` of it, by the team kernel
-// (team.hip).  done: false if its workgroups did not all come to run at once
-// (results of these frames are then not to be used).
+static int team_buffers(gf2l_ctx *ctx, const CodeView &cv, const TeamArgs &a, uint32_t F) {
+    return ensure_buffers(ctx, F, a.team > 1 ? (size_t)cv.nbe * cv.zp * a.teams : 0, 0, (size_t)cv.nb * cv.zp * a.teams,
+                          (size_t)a.teams * kTeamSyncStride, a.llr_words);
+}
+
+// Plain min-sum of a batch of F frames, or of the `count` frames of it in a
+// device list, by the team kernel (team.hip).  done: false if its workgroups did
+// not all come to run at once (results of these frames are then not to be used).
+// With a list, fewer and larger teams than the workspace holds: their messages,
+// beliefs and counters fit.
 static int decode_team(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
-                       TeamArgs &a, const std::vector<uint32_t> *only, uint64_t *d_msg, uint32_t *d_iters,
+                       TeamArgs &a, uint32_t *list, uint32_t count, uint64_t *d_msg, uint32_t *d_iters,
                        uint8_t *d_conv, uint8_t *d_synd, bool &done) {
     const CodeView &cv = code->view;
     hipStream_t s = ctx->stream;
-    const size_t sync = (size_t)a.teams * kTeamSyncStride;
-    int rc = ensure_buffers(ctx, F, a.team > 1 ? (size_t)cv.nbe * cv.zp * a.teams : 0, 0,
-                            (size_t)cv.nb * cv.zp * a.teams, sync,
-                            a.llr_words);
-    if (rc != GF2L_OK) return rc;
     Workspace &ws = ctx->ws;
-    GF2L_HIP(ctx, launch_clear_words(reinterpret_cast<uint32_t *>(ws.hb), (uint32_t)(2 * sync), s));
+    if (list) {  // in the workspace, which was sized for the whole batch and stays
+        if (ws.cap_llr < a.llr_words || ws.cap_c2v < (size_t)cv.nbe * cv.zp * a.teams) return GF2L_OK;
+    } else {
+        const int rc = team_buffers(ctx, cv, a, F);
+        if (rc != GF2L_OK) return rc;
+    }
+    GF2L_HIP(ctx, launch_clear_words(reinterpret_cast<uint32_t *>(ws.hb), 2 * a.teams * kTeamSyncStride, s));
     GF2L_HIP(ctx, launch_clear_words(ws.counts, 2, s));
     a.cv = cv;
     a.llr = d_llr;
-    a.frames = only ? (uint32_t)only->size() : F;
-    if (only) {
-        GF2L_HIP(ctx, hipMemcpyAsync(ws.lists, only->data(), only->size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        a.list = ws.lists;
-    }
+    a.frames = count;
+    a.list = list;
     a.max_it = max_it;
     a.llr_own = ws.llr_perm;
     a.msg = ws.c2v;
@@ -317,29 +322,24 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         TeamArgs team{};
         bool done = false;
         if (use_team(ctx, code, F, max_it, team)) {
-            std::vector<uint32_t> rest;
-            const bool first = team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3;
-            if (first) {
+            uint32_t *list = nullptr, count = F;
+            if (team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3 && max_it > 1) {
                 // Teams take several frames each: the first iteration by the
                 // state kernels, which are faster at it (202 error-free frames
-                // of DVB-T2 normal r 3/5: 292 us with the iterations they queue
-                // behind it, 345 by teams; in noise the teams alone would take
-                // 3% to 16% less), then teams for the frames still running.
+                // of DVB-T2 normal r 3/5: 265 us, 345 by teams; in noise the
+                // teams alone would take 3% to 16% less), then teams for the
+                // frames still running.
                 int rc1 = ensure_workspace(ctx, cv, path, F);
+                if (rc1 == GF2L_OK) rc1 = team_buffers(ctx, cv, team, F);
                 if (rc1 == GF2L_OK)
                     rc1 = run_hbm(ctx, cv, path, ctx->ws, d_llr, F, 1, nullptr, 0, false, d_msg, d_iters, d_conv, d_synd,
-                                  nullptr, nullptr, nullptr, 0, nullptr, nullptr, false, nullptr);
-                if (rc1 != GF2L_OK || max_it == 1) return rc1;
-                std::vector<uint8_t> conv(F);
-                GF2L_HIP(ctx, hipMemcpyAsync(conv.data(), d_conv, F, hipMemcpyDeviceToHost, s));
-                GF2L_HIP(ctx, hipStreamSynchronize(s));
-                for (uint32_t f = 0; f < F; ++f)
-                    if (!conv[f]) rest.push_back(f);
-                if (rest.empty()) return GF2L_OK;
-                use_team(ctx, code, (uint32_t)rest.size(), max_it, team);  // sizes for fewer frames
+                                  nullptr, nullptr, nullptr, 0, nullptr, nullptr, false, nullptr, &count);
+                if (rc1 != GF2L_OK || count == 0) return rc1;
+                list = ctx->ws.lists + ctx->ws.cap_frames;
+                use_team(ctx, code, count, max_it, team);  // sizes for fewer frames
             }
-            const int rct = decode_team(ctx, code, d_llr, F, max_it, team, first ? &rest : nullptr, d_msg, d_iters,
-                                        d_conv, d_synd, done);
+            const int rct = decode_team(ctx, code, d_llr, F, max_it, team, list, count, d_msg, d_iters, d_conv, d_synd,
+                                        done);
             if (rct != GF2L_OK || done) return rct;
         }
     }
@@ -429,7 +429,7 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             uint32_t max_it, const float *d_w, uint32_t fb_it, bool fb_continue, uint64_t *d_msg,
             uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd, uint8_t *d_fb, float *h_trace_c2v,
             float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs,
-            const std::vector<uint32_t> *only) {
+            const std::vector<uint32_t> *only, uint32_t *left) {
     hipStream_t s = ctx->stream;
     const size_t E = (size_t)cv.nbe * cv.z;
     gf2l::Profile &pf = ctx->prof;
@@ -484,7 +484,7 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             a.it = cont ? max_it + it : it;
             a.cur = g & 1u;
             a.it_report = (phase == 0 ? 0 : max_it) + it;
-            a.last = it == n_it && final_phase;
+            a.last = it == n_it && final_phase && !left;
             a.fb_phase = (int)phase;
             a.w_prev = (w && it >= 2) ? w + (size_t)(it - 2) * cv.nbe : nullptr;
             a.w_cur = w ? w + (size_t)(it - 1) * cv.nbe : nullptr;
@@ -552,6 +552,7 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             }
             running = ws.h_count[ph ? queued - 1 : 0];
             queued = 0;
+            if (left) *left = running;
             if (running == 0) {
                 const uint32_t done = it - 1;  // the iteration that retired the last frame
                 if (phase == 0 && h_trace_c2v)

@@ -359,12 +359,14 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
 // caller has prepared (gf2ldpc_api.hip); allocates nothing.  Used by
 // decode_device after growing the context's workspace and by the
 // no-allocation entry point over its static scratch array.  only (may be
-// null): the frames to decode, of the F the buffers hold.
+// null): the frames to decode, of the F the buffers hold.  left (may be null;
+// one plain iteration): frames that iteration leaves running are not retired,
+// their number goes to *left, their list to ws.lists + ws.cap_frames.
 int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const float *d_llr, uint32_t F,
             uint32_t max_it, const float *d_w, uint32_t fb_it, bool fb_continue, uint64_t *d_msg,
             uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd, uint8_t *d_fb, float *h_trace_c2v,
             float *h_trace_bel, uint32_t trace_iters, float *d_tc, float *d_tb, bool graphs = true,
-            const std::vector<uint32_t> *only = nullptr);
+            const std::vector<uint32_t> *only = nullptr, uint32_t *left = nullptr);
 // Decoder path (GF2L_PATH_*) the context would run a quasi-cyclic code on,
 // or -1 when a forced path cannot run it.
 int resolve_path(const gf2l_ctx *ctx, const CodeView &cv);
