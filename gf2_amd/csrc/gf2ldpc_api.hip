@@ -136,7 +136,7 @@ static bool use_team(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F, uin
     // DVB codes: faster than the state kernels at every batch size and rate
     // (normal r 1/2: 1 frame 1013 -> 245 us, 202 frames 4.23 -> 3.61 ms, 1000
     // frames 14.8 -> 14.2 ms; r 2/3: 1000 frames 16.1 -> 11.4 ms; short r 1/2:
-    // 1000 frames 5.03 -> 3.42 ms).
+    // 1000 frames 5.05 -> 3.27 ms).
     if (!code->flood.nd) return true;
     // Codes of the whole-frame kernel.  Those with two of its workgroups to a
     // compute unit (N = 16200, r 0.44): teams of four or more win (1 frame 255 ->
