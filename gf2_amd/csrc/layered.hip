@@ -259,9 +259,12 @@ __device__ __forceinline__ float flip(float x, uint32_t s) { return __uint_as_fl
 // w * (+-m) is computed as +-(w * m) (IEEE multiplication: the same value).
 // TAPE (training forward): the new state goes to the tape with the second
 // argmin and the input signs at both argmins; no hard decisions.
+// wild (decoding): NaN from here on when the parity column that the layer
+// completes is not finite.
 template <int D, bool TAPE>
 __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFrame &S, uint32_t br, uint32_t e0,
-                                            bool cin, bool last, const uint3 o, const float bo, float &carry) {
+                                            bool cin, bool last, const uint3 o, const float bo, float &carry,
+                                            float &wild) {
     static_assert(D >= 2 && D <= 8, "the staircase layer's sign rule needs 2 <= D <= 8");
     const CodeView &cv = a.cv;
     uint32_t cb[D], sh[D];
@@ -316,7 +319,8 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
     // Decoding takes the signs as sign bits, shifted in one instruction an
     // input: a -0.0 input counts as negative then, which turns the sign of
     // messages of magnitude zero only (its own message does not depend on it),
-    // and no zero's sign reaches a decision, a count or a nonzero belief.
+    // and no zero's sign reaches a decision, a count or a nonzero belief.  (A
+    // NaN's sign bit does count where it should not: see wild.)
     if constexpr (!TAPE)
 #pragma unroll
         for (int p = D - 1; p >= 0; --p) lt = __builtin_amdgcn_alignbit(lt, __float_as_uint(x[p]), 31u);
@@ -346,6 +350,7 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
             if (last && !TAPE) {
                 const uint64_t m = __ballot(v < 0.0f);
                 if (lane == 0) S.hb[(cv.nb - 1) * cv.zw + wave] = m;
+                wild = __builtin_fmaf(v, 0.0f, wild);
             }
         } else if (p == D - 2) {
             // column kb+br-1, final for this iteration (block-row 0: an
@@ -356,6 +361,7 @@ __device__ __forceinline__ void stair_layer(const LayeredArgs &a, const StairFra
                 if constexpr (!TAPE) {
                     const uint64_t m = __ballot(v < 0.0f);
                     if (lane == 0) S.hb[(S.kb + br - 1) * cv.zw + wave] = m;
+                    wild = __builtin_fmaf(v, 0.0f, wild);
                 }
             } else {
                 lds_st(ad[p], v);
@@ -427,6 +433,58 @@ __device__ __forceinline__ uint32_t mask_slice(uint64_t m0, uint64_t m1, uint64_
     return (uint32_t)((lo >> o) | (o ? hi << (64u - o) : 0ull));
 }
 
+// One iteration of a frame, layer by layer, by the comparisons of the general
+// kernel (CheckAcc): for the rare frames with values that are not finite.  A
+// function of its own, so that its registers are not the kernel's.
+__device__ __attribute__((noinline)) void stair_iteration(const lds_u32 *tab, const lds_u64 *re, const lds_u32 *rp,
+                                                          float *gb, uint3 *st, uint32_t z, uint32_t zp, uint32_t mb,
+                                                          uint32_t kb, bool first) {
+    constexpr int DMAX = 8;
+    const uint32_t i = threadIdx.x;  // < z
+    for (uint32_t br = 0; br < mb; ++br) {
+        const uint32_t e0 = rp[br], d = rp[br + 1] - e0;
+        const uint3 o = first ? make_uint3(0, 0, 0) : st[br * zp + i];
+        float x[DMAX], m1 = __builtin_inff(), m2 = __builtin_inff();
+        uint32_t idx = 0, lt = 0;
+#pragma unroll
+        for (int p = 0; p < DMAX; ++p) {
+            if (p >= (int)d) continue;
+            const lds_u32 *r = tab + 4 * (e0 + p);
+            const uint32_t col = (uint32_t)re[e0 + p];
+            const float b = col < kb ? lds_ld(r[0] + 4u * wrap_add(i, r[1], z)) : gb[col * zp + i];
+            const float mag = __uint_as_float((uint32_t)p == (o.z & 31u) ? o.y : o.x);
+            x[p] = b - flip(__uint_as_float(r[3]) * mag, (o.z >> (5 + p)) & 1u);
+            const float v = fabsf(x[p]);
+            const bool lt1 = v < m1, lt2 = v < m2;
+            m2 = lt1 ? m1 : (lt2 ? v : m2);
+            m1 = lt1 ? v : m1;
+            idx = lt1 ? (uint32_t)p : idx;
+            lt |= (x[p] < 0.0f ? 1u : 0u) << p;
+        }
+        const uint32_t sg = ((__popc(lt) & 1u) ? (1u << d) - 1u : 0u) ^ lt;
+#pragma unroll
+        for (int p = 0; p < DMAX; ++p) {
+            if (p >= (int)d) continue;
+            const lds_u32 *r = tab + 4 * (e0 + p);
+            const uint32_t col = (uint32_t)re[e0 + p];
+            const float v = x[p] + flip(__uint_as_float(r[2]) * ((uint32_t)p == idx ? m2 : m1), (sg >> p) & 1u);
+            if (col < kb)
+                lds_st(r[0] + 4u * wrap_add(i, r[1], z), v);
+            else
+                gb[col * zp + i] = v;
+        }
+        st[br * zp + i] = make_uint3(__float_as_uint(m1), __float_as_uint(m2), idx | (sg << 5));
+        __syncthreads();
+    }
+}
+
+// A frame in which some belief was not finite after an iteration is decoded
+// again, each layer by the rule's comparisons (stair_iteration).  Within an
+// iteration such a belief stays one (x = b - old and x + message are infinite or
+// NaN again), so two instructions a column and iteration find it.  4096 frames of
+// N=64800: 11.12 -> 11.25 ms; one instruction more for every input, in the chain
+// of every layer, 11.53.
+//
 // TAPE: the training forward.  All T iterations; the tape of an iteration is
 // also what the next one reads its old states and parity beliefs from.
 // N=64800, 256 frames, 10 iterations: 0.86 ms against 3.04 ms for the general
@@ -494,7 +552,7 @@ __global__ void __launch_bounds__(512) lnms_stair_kernel(LayeredArgs a) {
         // unrestricted)
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
-        float carry = 0.0f;
+        float carry = 0.0f, wild = 0.0f;
         int conv = 0;
         uint32_t t = 1, br = 0, e0 = 0;  // br: first block-row of the group, e0: its first edge
         for (;;) {
@@ -520,9 +578,9 @@ __global__ void __launch_bounds__(512) lnms_stair_kernel(LayeredArgs a) {
                 const bool cin = u > 0 || br > 0;      // a constant in all but the first copy
                 const bool last = u == P - 1 && wrap;  // false in all but the last copy
                 if (hi)
-                    stair_layer<DH, TAPE>(a, S, r, e0, cin, last, sst[u], sbo[u], carry);
+                    stair_layer<DH, TAPE>(a, S, r, e0, cin, last, sst[u], sbo[u], carry, wild);
                 else
-                    stair_layer<DH - 1, TAPE>(a, S, r, e0, cin, last, sst[u], sbo[u], carry);
+                    stair_layer<DH - 1, TAPE>(a, S, r, e0, cin, last, sst[u], sbo[u], carry, wild);
                 e0 += hi ? DH : DH - 1;
                 // loaded whether or not it will be used (past iteration T): in
                 // bounds, one definition per slot; wave-uniform row bases, so
@@ -552,8 +610,10 @@ __global__ void __launch_bounds__(512) lnms_stair_kernel(LayeredArgs a) {
                 const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
                 if constexpr (!TAPE) {
                     for (uint32_t c = 0; c < kb; ++c) {
-                        const uint64_t m = __ballot(s_bel[c * cv.z + i] < 0.0f);
+                        const float b = s_bel[c * cv.z + i];
+                        const uint64_t m = __ballot(b < 0.0f);
                         if (lane == 0) s_hb[c * cv.zw + wave] = m;
+                        wild = __builtin_fmaf(b, 0.0f, wild);
                     }
                     lds_barrier();
                     if (!stair_unsat(cv, s_hb, s_rp, s_re, s_bad)) {
@@ -576,6 +636,30 @@ __global__ void __launch_bounds__(512) lnms_stair_kernel(LayeredArgs a) {
             }
         }
         if constexpr (TAPE) continue;
+        if (__syncthreads_or(wild != 0.0f)) {  // again, with the comparisons themselves
+            for (uint32_t c = 0; c < cv.nb; ++c) {
+                const float l = S.llr[c * cv.z + i];
+                if (c < kb)
+                    s_bel[c * cv.z + i] = l;
+                else
+                    S.gb[c * cv.zp + i] = l;
+            }
+            for (t = 1, conv = 0;; ++t) {
+                for (uint32_t e = i; e < cv.nbe; e += cv.z) {
+                    s_tab[4 * e + 3] = t > 1 ? __float_as_uint(a.w[(size_t)(t - 2) * cv.nbe + e]) : 0u;
+                    s_tab[4 * e + 2] = __float_as_uint(a.w[(size_t)(t - 1) * cv.nbe + e]);
+                }
+                __syncthreads();
+                stair_iteration(s_tab, s_re, s_rp, S.gb, S.st, cv.z, cv.zp, cv.mb, kb, t == 1);
+                for (uint32_t c = 0; c < cv.nb; ++c) {
+                    const uint64_t m = __ballot((c < kb ? s_bel[c * cv.z + i] : S.gb[c * cv.zp + i]) < 0.0f);
+                    if ((i & 63u) == 0) s_hb[c * cv.zw + (i >> 6)] = m;
+                }
+                __syncthreads();
+                conv = !stair_unsat(cv, s_hb, s_rp, s_re, s_bad);
+                if (conv || t == a.T) break;
+            }
+        }
         const uint32_t its = conv ? t : a.T;
         if (threadIdx.x == 0) atomicAdd(a.ctr + 1, its);
         if (conv || !a.fallback) {
