@@ -294,8 +294,13 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
     }
     if (path < 0) return fail(ctx, GF2L_ERR_UNSUPPORTED, "the forced decoder path cannot run this code");
     if (path == gf2l::kLds && !d_w && !d_fb && !h_trace_c2v && use_small_kernel(ctx, code)) {
+        // A launch that is being recorded takes its frames at a fixed stride:
+        // its replays may run beside each other and beside this context's own
+        // launches, which share the frame counter one after another.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        GF2L_HIP(ctx, hipStreamIsCapturing(s, &capture));
         GF2L_HIP(ctx, launch_small(cv, code->small_threads, d_llr, F, max_it, d_msg, d_iters, d_conv, d_synd,
-                                   ctx->d_small, ctx->num_cus, s));
+                                   capture == hipStreamCaptureStatusNone ? ctx->d_small : nullptr, ctx->num_cus, s));
         return GF2L_OK;
     }
     if (path == gf2l::kLds) {
