@@ -105,7 +105,9 @@ struct Channel {
         const double ebn0 = (double)lo + ((double)hi - (double)lo) * u;
         const double s2 = 1.0 / (2.0 * rate * pow(10.0, ebn0 / 10.0));
         one = 2.0 / s2;
-        noise = sqrt(s2) * one;
+        // no noise is left in an infinite LLR (3,082 dB up: s2 is 0, or 2 / s2
+        // past the largest double)
+        noise = one < __builtin_inf() ? sqrt(s2) * one : 0.0;
     }
     __device__ double2 pair(const uint32_t o[4]) const {
         const double u1 = ((double)o[0] + 0.5) * (1.0 / 4294967296.0);
