@@ -130,22 +130,41 @@ static bool use_small_kernel(const gf2l_ctx *ctx, const gf2l_code *code) {
 // Whether a plain batch runs the team kernel, and its sizes.
 static bool use_team(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F, uint32_t max_it, TeamArgs &a) {
     const int mode = ctx->tune.frame_kernel;
-    if (mode == 1 || mode == 2 || !team_shape(code->view, F, max_it, ctx->num_cus, ctx->lds_limit, a)) return false;
+    const CodeView &cv = code->view;
+    if (mode == 1 || mode == 2 || !team_shape(cv, F, max_it, ctx->num_cus, ctx->lds_limit, a)) return false;
     if (mode >= 3) return true;
     if (ctx->path != gf2l::kAuto || ctx->tune.hbm_graph || ctx->prof.on) return false;
-    // DVB codes: faster than the state kernels at every batch size and rate
-    // (normal r 1/2: 1 frame 1013 -> 245 us, 202 frames 4.23 -> 3.61 ms, 1000
-    // frames 14.8 -> 14.2 ms; r 2/3: 1000 frames 16.1 -> 11.4 ms; short r 1/2:
-    // 1000 frames 5.05 -> 3.27 ms).
-    if (!code->flood.nd) return true;
-    // Codes of the whole-frame kernel.  Those with two of its workgroups to a
-    // compute unit (N = 16200, r 0.44): teams of four or more win (1 frame 255 ->
-    // 137 us, 64 frames 386 -> 306 us), teams of two lose (100 frames 430 -> 541
-    // us).  Longer ones: wherever every frame has a team at once (N = 64800: 24
-    // frames 1446 -> 480 us, 85 frames 2.71 -> 2.42 ms, at r 2/3 128 frames 1.35
-    // -> 1.33 ms; with a second turn 128 frames at r 1/2 2.72 -> 2.92 ms).
-    if (flood_bytes(code->view, code->flood) <= 80 * 1024) return a.team >= 4;
-    return F <= a.teams && a.team > 1;
+    // Teams take turns at a batch larger than they are; a last turn that is
+    // nearly empty costs as much as a full one.  full: at least three quarters of
+    // the compute units have work over all turns.
+    const uint64_t cus = (uint64_t)ctx->num_cus, room = cus / a.team, turns = (F + room - 1) / room;
+    const bool full = 4ull * F * a.team >= 3 * turns * cus;
+    // Whole-frame kernel's codes.  Those with two of its workgroups to a compute
+    // unit (N = 16200, r 0.44): teams of four or more win (1 frame 255 -> 137 us,
+    // 64 frames 386 -> 306 us), teams of two lose (100 frames 430 -> 541 us).
+    // Longer ones: where every frame has a team at once (N = 64800: 24 frames 1446
+    // -> 480 us, at r 2/3 128 frames 3443 -> 3100 us, but 86 frames in teams of
+    // two 2595 -> 2750 us; with a second turn 128 frames at r 1/2 2.72 -> 2.92 ms).
+    if (code->flood.nd) {
+        if (flood_bytes(cv, code->flood) <= 80 * 1024) return a.team >= 4;
+        return turns == 1 && a.team > 1 && full;
+    }
+    // The other codes against the STATE kernels.  One workgroup a frame: at every
+    // batch size (DVB-T2 normal r 5/6 1000 frames 14.2 -> 8.6 ms, N = 24000 with
+    // z = 500 4096 frames 15.4 -> 11.7 ms).  Larger teams: wherever every frame has
+    // one at once (N = 64800: 1 frame 635 -> 163 us, 85 frames 1532 -> 1318 us).
+    if (a.team == 1 || turns == 1) return true;
+    // Several turns of larger teams: where the STATE kernels are slow, in full
+    // turns.  They hold back with many messages a variable (DVB-T2 normal r 2/3,
+    // columns of 13: 1000 frames 22.7 -> 15.0 ms, 500 11.2 -> 8.0, but 150 frames,
+    // a second turn of 22, 3.82 -> 3.86 ms) and with short block-rows (N = 64768
+    // with z = 128, 256 frames 3.94 -> 3.03 ms, z = 64 6.13 -> 3.18, and there also
+    // with short turns: 90 frames 2.66 -> 1.67 ms).  Otherwise they catch up with
+    // the number of frames (DVB-T2 normal r 1/2, columns of 8: 170 frames 4.36 ->
+    // 3.44 ms, 500 10.2 -> 9.1, 1000 at 0.6 dB more 9.4 -> 10.0; N = 64800 with
+    // z = 360 and no staircase: 1024 frames 10.4 -> 11.1 ms).
+    if (cv.z <= 64) return true;
+    return full && (cv.max_dv > 8 || cv.z <= 128 || (cv.dvb_q && turns <= 6));
 }
 
 // Plain min-sum by the whole-frame kernel (flood.hip): results of every frame
@@ -328,24 +347,28 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         bool done = false;
         if (use_team(ctx, code, F, max_it, team)) {
             uint32_t *list = nullptr, count = F;
-            if (team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3 && max_it > 1) {
-                // Teams take several frames each: the first iteration by the
-                // state kernels, which are faster at it (202 error-free frames
-                // of DVB-T2 normal r 3/5: 265 us, 345 by teams; in noise the
-                // teams alone would take 3% to 16% less), then teams for the
-                // frames still running.
+            bool fits = true;
+            if (cv.dvb_q && team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3 && max_it > 1) {
+                // DVB codes whose teams take several frames each: the first
+                // iteration by the state kernels, which are faster at it (202
+                // error-free frames of DVB-T2 normal r 3/5: 265 us, 345 by teams;
+                // in noise the teams alone would take 3% to 16% less), then teams
+                // for the frames still running.
                 int rc1 = ensure_workspace(ctx, cv, path, F);
                 if (rc1 == GF2L_OK) rc1 = team_buffers(ctx, cv, team, F);
                 if (rc1 == GF2L_OK)
-                    rc1 = run_hbm(ctx, cv, path, ctx->ws, d_llr, F, 1, nullptr, 0, false, d_msg, d_iters, d_conv, d_synd,
-                                  nullptr, nullptr, nullptr, 0, nullptr, nullptr, false, nullptr, &count);
+                    rc1 = run_hbm(ctx, cv, path, ctx->ws, d_llr, F, max_it, nullptr, 0, false, d_msg, d_iters, d_conv,
+                                  d_synd, nullptr, nullptr, nullptr, 0, nullptr, nullptr, false, nullptr, &count);
                 if (rc1 != GF2L_OK || count == 0) return rc1;
                 list = ctx->ws.lists + ctx->ws.cap_frames;
-                use_team(ctx, code, count, max_it, team);  // sizes for fewer frames
+                // sizes for fewer frames
+                fits = team_shape(cv, count, max_it, ctx->num_cus, ctx->lds_limit, team);
             }
-            const int rct = decode_team(ctx, code, d_llr, F, max_it, team, list, count, d_msg, d_iters, d_conv, d_synd,
-                                        done);
-            if (rct != GF2L_OK || done) return rct;
+            if (fits) {
+                const int rct = decode_team(ctx, code, d_llr, F, max_it, team, list, count, d_msg, d_iters, d_conv,
+                                            d_synd, done);
+                if (rct != GF2L_OK || done) return rct;
+            }
         }
     }
     std::vector<uint32_t> left;  // frames the whole-frame kernel leaves to the general ones
@@ -489,7 +512,7 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             a.it = cont ? max_it + it : it;
             a.cur = g & 1u;
             a.it_report = (phase == 0 ? 0 : max_it) + it;
-            a.last = it == n_it && final_phase && !left;
+            a.last = it == n_it && final_phase;
             a.fb_phase = (int)phase;
             a.w_prev = (w && it >= 2) ? w + (size_t)(it - 2) * cv.nbe : nullptr;
             a.w_cur = w ? w + (size_t)(it - 1) * cv.nbe : nullptr;
@@ -539,7 +562,7 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             // first iteration of a phase that continues in a graph is read
             // back too (the graph starts a batch)
             const bool to_graph = use_graph && final_phase && !w && it + 1 <= n_it;
-            const bool readback = queued + 1 >= batch || (it == n_it && final_phase) || to_graph;
+            const bool readback = queued + 1 >= batch || (it == n_it && final_phase) || to_graph || left;
             if (ph || readback)
                 GF2L_HIP(ctx, hipMemcpyAsync(ws.h_count + (ph ? queued : 0), ws.counts + ((g + 1) & 1u),
                                              sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -557,7 +580,14 @@ int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const fl
             }
             running = ws.h_count[ph ? queued - 1 : 0];
             queued = 0;
-            if (left) *left = running;
+            if (left) {
+                // frames that one iteration has done are a sign of a quiet
+                // channel: a few more iterations here cost less than a new start
+                const bool quiet = 8ull * (F - running) >= F;
+                *left = quiet ? 0 : running;
+                if (!quiet) return GF2L_OK;
+                left = nullptr;
+            }
             if (running == 0) {
                 const uint32_t done = it - 1;  // the iteration that retired the last frame
                 if (phase == 0 && h_trace_c2v)

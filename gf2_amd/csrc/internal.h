@@ -360,8 +360,9 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
 // decode_device after growing the context's workspace and by the
 // no-allocation entry point over its static scratch array.  only (may be
 // null): the frames to decode, of the F the buffers hold.  left (may be null;
-// one plain iteration): frames that iteration leaves running are not retired,
-// their number goes to *left, their list to ws.lists + ws.cap_frames.
+// plain, max_it above 1): where the first iteration is done with less than an
+// eighth of the frames, the call ends there, with the number of the others in
+// *left and their list at ws.lists + ws.cap_frames; else *left is 0.
 int run_hbm(gf2l_ctx *ctx, const CodeView &cv, int path, Workspace &ws, const float *d_llr, uint32_t F,
             uint32_t max_it, const float *d_w, uint32_t fb_it, bool fb_continue, uint64_t *d_msg,
             uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd, uint8_t *d_fb, float *h_trace_c2v,
