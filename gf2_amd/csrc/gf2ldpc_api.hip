@@ -348,7 +348,7 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
         if (use_team(ctx, code, F, max_it, team)) {
             uint32_t *list = nullptr, count = F;
             bool fits = true;
-            if (cv.dvb_q && team.team > 1 && F > team.teams && ctx->tune.frame_kernel < 3 && max_it > 1) {
+            if (cv.dvb_q && team.team > 1 && F > team.teams && ctx->tune.frame_kernel != 3 && max_it > 1) {
                 // DVB codes whose teams take several frames each: the first
                 // iteration by the state kernels, which are faster at it (202
                 // error-free frames of DVB-T2 normal r 3/5: 265 us, 345 by teams;

@@ -194,9 +194,11 @@ int gf2l_set_check_rule(gf2l_ctx *ctx, int rule);
  *                        GF2L_TUNE_LDS_GROUPS or GF2L_TUNE_HBM_GRAPH set; no
  *                        teams while profiling), 1 never, 2 a workgroup per
  *                        frame wherever the code allows it, 3 teams wherever
- *                        the code allows it, 4 as 3, but a team whose
- *                        workgroups do not meet at once leaves the batch to
- *                        the general kernels (otherwise after 0.3 ms). */
+ *                        the code allows it, 4 as 3, but with the state
+ *                        kernels' first iteration for DVB batches larger than
+ *                        their teams (as in 0), and a team whose workgroups do
+ *                        not meet at once leaves the batch to the general
+ *                        kernels (otherwise after 0.3 ms). */
 #define GF2L_TUNE_WG_PER_CU 1
 #define GF2L_TUNE_XCD_MAP 2
 #define GF2L_TUNE_GRAPH_ITERS 3

@@ -11,7 +11,7 @@ from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
 
-GENERAL = 1
+GENERAL, TEAM_NO_WAIT = 1, 4
 
 
 @pytest.fixture(scope="module")
@@ -77,7 +77,8 @@ def test_dvb_batches_of_several_turns(ctx, rate, counts, quiet):
     llr[rng.random(max(counts)) < quiet] = 10.0
     want = oc.decode_batch(llr[:4], 12, threads=8)
     for count in counts:
-        print("[gpu-case] team turns", rate, count, quiet, flush=True)
-        got = decode(ctx, code, llr[:count], 12, 0)
-        same(got, decode(ctx, code, llr[:count], 12, GENERAL), (rate, count, quiet))
-        same([x[:4] for x in got], want, (rate, count, quiet, "oracle"))
+        for mode in (0, TEAM_NO_WAIT):  # with and without teams that leave after the first iteration
+            print("[gpu-case] team turns", rate, count, quiet, mode, flush=True)
+            got = decode(ctx, code, llr[:count], 12, mode)
+            same(got, decode(ctx, code, llr[:count], 12, GENERAL), (rate, count, quiet, mode))
+            same([x[:4] for x in got], want, (rate, count, quiet, mode, "oracle"))
