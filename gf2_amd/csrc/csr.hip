@@ -72,8 +72,9 @@ vn_csr_kernel(CsrView cv, const uint32_t *__restrict__ list, const uint32_t *__r
 
 // One workgroup per frame: syndrome from the linear hard-decision words, then
 // retire (first k bits are the message) or keep the frame running.  A frame's
-// checks are dependent table and bit lookups: sixteen waves hide what one wave
-// waited for (4,500 checks, 500 frames: 4.01 -> 2.57 ms for the decode).
+// checks are dependent table and bit lookups: up to sixteen waves, as many as have
+// checks, hide what one wave waited for (4,500 checks, 500 frames: 4.01 -> 2.57 ms
+// for the decode).
 constexpr uint32_t kSynThreads = 1024;
 __global__ void __launch_bounds__(kSynThreads)
 syn_csr_kernel(CsrView cv, const uint32_t *__restrict__ list, const uint32_t *__restrict__ count_ptr,
@@ -141,21 +142,33 @@ constexpr uint32_t kGroupThreads = 512;  // of the check and variable passes
 
 // Workgroup split (workgroup b runs on XCD b % 8): whole rounds of eight groups
 // go one group to an XCD, whose L2 then serves the repeated reads of the
-// group's beliefs; the rows of the up to seven groups left over are spread over
-// the chip (one group of 8,000 checks on one XCD took 60 us an iteration).
+// group's beliefs; there `share` workgroups take a group, and where a code has
+// fewer rows than the XCD's workgroups have waves several groups run beside each
+// other (one after the other, 65,536 frames of n = 64 took 5.0 ms for seven
+// iterations, now 0.9; a million of n = 7 18.3, now 0.5).  The rows of the up to
+// seven groups left over are spread over the chip (one group of 8,000 checks on
+// one XCD took 60 us an iteration), each over its own part of it (split) where
+// every row finds a wave there: 256 error-free frames of n = 300 58 -> 39 us.
 // Calls f(group, first row, row stride, this workgroup's place among those of
 // the group, their number).
+struct GroupSplit {
+    uint32_t share, split;
+};
 template <typename F>
-__device__ __forceinline__ void each_group(uint32_t groups, F &&f) {
-    const uint32_t x = blockIdx.x & 7u, per = blockDim.x >> 6;
-    const uint32_t wave = (blockIdx.x >> 3) * per + uni(threadIdx.x >> 6), waves = (gridDim.x >> 3) * per;
-    const uint32_t full = groups >> 3, turns = full + (groups & 7u);
-    for (uint32_t t = 0; t < turns; ++t) {
-        const bool spread = t >= full;
-        const uint32_t g = spread ? 7u * full + t : 8u * t + x;
-        f(g, spread ? 8u * wave + x : wave, spread ? 8u * waves : waves, spread ? blockIdx.x : blockIdx.x >> 3,
-          spread ? gridDim.x : gridDim.x >> 3);
+__device__ __forceinline__ void each_group(uint32_t groups, GroupSplit sp, F &&f) {
+    const uint32_t share = sp.share;
+    const uint32_t x = blockIdx.x & 7u, b = blockIdx.x >> 3, per = blockDim.x >> 6, wave = uni(threadIdx.x >> 6);
+    const uint32_t full = groups >> 3, beside = (gridDim.x >> 3) / share, at = b / share, place = b - at * share;
+    if (at < beside)
+        for (uint32_t t = at; t < full; t += beside) f(8u * t + x, place * per + wave, share * per, place, share);
+    const uint32_t left = groups & 7u;
+    if (left && sp.split) {
+        const uint32_t part = gridDim.x / left, g = blockIdx.x / part, p = blockIdx.x - g * part;
+        if (g < left) f(8u * full + g, p * per + wave, part * per, p, part);
+        return;
     }
+    for (uint32_t g = 8u * full; g < groups; ++g)
+        f(g, 8u * (b * per + wave) + x, gridDim.x * per, blockIdx.x, gridDim.x);
 }
 
 // Check messages of one check for 64 frames: CheckAcc's rule.  Up to 8 inputs
@@ -222,11 +235,11 @@ __device__ __forceinline__ uint64_t group_or(uint64_t v, uint64_t *red) {
 // it - 1 that it reads.  FIRST: beliefs are the LLRs, no old messages.
 template <int MAXD, bool FIRST>
 __global__ void __launch_bounds__(kGroupThreads)
-cn_group_kernel(CsrView cv, uint32_t groups, GroupState gs, float *__restrict__ c2v, const float *__restrict__ belief) {
+cn_group_kernel(CsrView cv, uint32_t groups, GroupSplit sp, GroupState gs, float *__restrict__ c2v, const float *__restrict__ belief) {
     const uint32_t lane4 = 4u * (threadIdx.x & 63u);
     if (blockIdx.x == 0 && threadIdx.x == 0) *gs.running = 0;
     __shared__ uint64_t red[kGroupThreads / 64];
-    each_group(groups, [&](uint32_t g, uint32_t r0, uint32_t step, uint32_t slot, uint32_t) {
+    each_group(groups, sp, [&](uint32_t g, uint32_t r0, uint32_t step, uint32_t slot, uint32_t) {
         if (ldc(gs.act_in + g) == 0) return;
         float *gc = c2v + (size_t)g * cv.nnz * 64u;
         const float *gb = belief + (size_t)g * cv.n * 64u;
@@ -266,13 +279,13 @@ cn_group_kernel(CsrView cv, uint32_t groups, GroupState gs, float *__restrict__ 
 // satisfied after iteration it - 1 (all frames in the pass after the last
 // iteration) leave with the hard decisions of that iteration.
 __global__ void __launch_bounds__(kGroupThreads)
-vn_group_kernel(CsrView cv, uint32_t groups, GroupState gs, const float *__restrict__ c2v, float *__restrict__ belief,
-                const float *__restrict__ llr, const uint64_t *__restrict__ hb_in, uint64_t *__restrict__ hb_out,
+vn_group_kernel(CsrView cv, uint32_t groups, GroupSplit sp, GroupState gs, const float *__restrict__ c2v,
+                float *__restrict__ belief, const float *__restrict__ llr, const uint64_t *__restrict__ hb_in, uint64_t *__restrict__ hb_out,
                 const uint32_t *__restrict__ map, uint32_t it, int last, uint64_t *__restrict__ msg,
                 uint32_t *__restrict__ iters, uint8_t *__restrict__ conv, uint8_t *__restrict__ synd) {
     const uint32_t lane = threadIdx.x & 63u, lane4 = 4u * lane;
     __shared__ uint64_t red[kGroupThreads / 64];
-    each_group(groups, [&](uint32_t g, uint32_t v0, uint32_t step, uint32_t, uint32_t slots) {
+    each_group(groups, sp, [&](uint32_t g, uint32_t v0, uint32_t step, uint32_t, uint32_t slots) {
         const uint64_t act = ldc(gs.act_in + g);
         if (act == 0) {  // uniform
             if (v0 == 0 && lane == 0) gs.act_out[g] = 0;
@@ -354,29 +367,42 @@ group_llr_kernel(const float *__restrict__ llr, float *__restrict__ out, uint32_
 }
 
 // Packing: the running lanes in order get new slots; src[new] = old slot.
-// One workgroup.
+// One workgroup, a stretch of the groups per wave: the waves count theirs, then
+// write from where the waves before them end, 64 masks in flight (one wave over
+// all groups waited for each of them).
 __global__ void __launch_bounds__(1024)
 group_pack_kernel(uint64_t *__restrict__ active, uint32_t groups, const uint32_t *__restrict__ map,
                   uint32_t *__restrict__ new_map, uint32_t *__restrict__ src, uint32_t total) {
-    __shared__ uint32_t s_base;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    __shared__ uint32_t s_sum[16];
+    const uint32_t lane = threadIdx.x & 63u, wave = uni(threadIdx.x >> 6);
     const uint32_t new_groups = (total + 63u) / 64u;
-    if (wave == 0) {
-        uint32_t base = 0;
-        for (uint32_t g = 0; g < groups; ++g) {
-            const uint64_t a = active[g];
+    const uint32_t stretch = (groups + 15u) / 16u, g0 = min(wave * stretch, groups), g1 = min(g0 + stretch, groups);
+    uint32_t sum = 0;
+    for (uint32_t g = g0 + lane; g < g1; g += 64u) sum += (uint32_t)__popcll(active[g]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += (uint32_t)__shfl_xor((int)sum, o, 64);
+    if (lane == 0) s_sum[wave] = sum;
+    __syncthreads();
+    uint32_t base = 0, used = 0;  // used: all of them (total, as the host read it)
+    for (uint32_t w = 0; w < 16u; ++w) {
+        base += w < wave ? s_sum[w] : 0u;
+        used += s_sum[w];
+    }
+    for (uint32_t gb = g0; gb < g1; gb += 64u) {
+        const uint64_t mine = gb + lane < g1 ? active[gb + lane] : 0ull;
+        const uint32_t count = min(64u, g1 - gb);
+        for (uint32_t k = 0; k < count; ++k) {
+            const uint64_t a = __shfl((unsigned long long)mine, (int)k, 64);
             if ((a >> lane) & 1ull) {
                 const uint32_t at = base + (uint32_t)__popcll(a & ((1ull << lane) - 1ull));
-                src[at] = g * 64u + lane;
-                new_map[at] = map[g * 64u + lane];
+                src[at] = (gb + k) * 64u + lane;
+                new_map[at] = map[(gb + k) * 64u + lane];
             }
             base += (uint32_t)__popcll(a);
         }
-        if (lane == 0) s_base = base;
     }
     __syncthreads();
     // the last group's free lanes repeat its last frame (masked off)
-    const uint32_t used = s_base;
     for (uint32_t t = used + threadIdx.x; t < new_groups * 64u; t += blockDim.x) {
         src[t] = src[used - 1u];
         new_map[t] = new_map[used - 1u];
@@ -406,19 +432,37 @@ group_move_kernel(const uint32_t *__restrict__ src, const float *__restrict__ in
 
 }  // namespace
 
-// Codes whose group arrays are indexed by 32-bit byte offsets run in groups, at
-// every batch size: two launches an iteration instead of three win where the
-// launches bound (one frame of n = 2,000: 280 -> 201 us, of n = 300,000: 3.59 ->
-// 3.39 ms), whole rows instead of gathered floats elsewhere (n = 9,000, 500
-// frames: 2.57 -> 0.89 ms against the kernels above).
-static bool use_groups(const CsrView &cv) {
+// Codes whose group arrays are indexed by 32-bit byte offsets run in groups: two
+// launches an iteration instead of three win where the launches bound (one frame
+// of n = 2,000: 280 -> 201 us, of n = 300,000: 3.59 -> 3.39 ms), whole rows instead
+// of gathered floats elsewhere (n = 9,000, 500 frames: 2.57 -> 0.89 ms against the
+// kernels above).  A single frame of up to 128 variables has nothing to win: 86
+// against 112 us for n = 7, 155 against 138 for n = 128.
+static bool use_groups(const CsrView &cv, uint32_t frames) {
+    if (frames == 1 && cv.n <= 128) return false;
     return cv.nnz > 0 && cv.m > 0 && cv.nnz < (1u << 20) && cv.n < (1u << 20);
 }
+static uint32_t group_grid_most(const gf2l_ctx *ctx) { return 8u * ((uint32_t)ctx->num_cus / 2u); }
+// Whether each of the last groups of a pass (fewer than eight) has its own part of
+// a full grid: every row of them finds a wave.
+static bool groups_split(const gf2l_ctx *ctx, const CsrView &cv, uint32_t groups) {
+    return (uint64_t)std::max(cv.m, cv.n) * (groups & 7u) <= (uint64_t)group_grid_most(ctx) * (kGroupThreads / 64u);
+}
 // Workgroups of a pass over `groups` groups: a multiple of 8, at most four to a
-// compute unit, and no more than the rows of a round of groups.
+// compute unit, and no more than the rows of a round of groups, or of all the
+// groups that are split (where they are not, more workgroups than one group needs
+// cost 10%: n = 3,000, 130 frames 250 -> 290 us).
 static uint32_t group_grid(const gf2l_ctx *ctx, const CsrView &cv, uint32_t groups) {
-    const uint32_t waves = kGroupThreads / 64u, rows = std::max(cv.m, cv.n) * ((groups + 7u) / 8u) / (groups < 8 ? 8 : 1);
-    return 8u * std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)ctx->num_cus / 2u, (rows + waves - 1u) / waves));
+    const uint64_t waves = kGroupThreads / 64u, one = std::max(cv.m, cv.n),
+                   rows = groups >= 8 ? one * ((groups + 7u) / 8u) : one * (groups_split(ctx, cv, groups) ? groups : 1u) / 8u;
+    return 8u * (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(group_grid_most(ctx) / 8u, (rows + waves - 1u) / waves));
+}
+// Workgroups of an XCD that share a group: four rows a wave, or fewer where there
+// are fewer groups than that leaves room for.
+static GroupSplit group_split(const gf2l_ctx *ctx, const CsrView &cv, uint32_t groups, uint32_t grid) {
+    const uint32_t waves = kGroupThreads / 64u, rows = std::max(cv.m, cv.n), rounds = std::max(1u, groups / 8u);
+    const uint32_t four = (rows + 4u * waves - 1u) / (4u * waves), one = (rows + waves - 1u) / waves;
+    return {std::min(grid / 8u, std::min(one, std::max(four, grid / 8u / rounds))), groups_split(ctx, cv, groups) ? 1u : 0u};
 }
 // Groups per pass: the workspace of a pass stays below 4 GiB (at least eight groups).
 static uint32_t groups_per_pass(const CsrView &cv) {
@@ -446,14 +490,20 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
     const uint32_t grid = group_grid(ctx, cv, groups);
     const uint32_t max_dc = code->view.max_dc;
     const uint32_t batch = (uint32_t)std::max(1, std::min(ctx->tune.graph_iters, kProfileSlots));
+    // Few frames of a short code: launches are all there is, so those that one
+    // iteration decodes are asked for at once (error-free: n = 2,000, 1 to 64 frames
+    // 75 -> 36 us, n = 64, 4,096 frames 77 -> 39; in noise n = 2,000, 16 frames 200
+    // -> 180; with 500 frames, or n = 9,000, the question costs 2% to 8% in noise).
+    const bool quick = cv.n <= 6000 && (uint64_t)cv.n * groups < 16000;
     // the pass after the last iteration takes its parities and retires the rest
     for (uint64_t it = 1; it <= (uint64_t)max_it + 1; ++it) {
         const uint32_t in = (it - 1) & 1u, out = it & 1u;
         const bool last = it > max_it;
         const GroupState gs{active[in], active[out], unsat, running};
+        const GroupSplit sp = group_split(ctx, cv, groups, grid);
         const float *b_in = it == 1 ? llr[cur] : bel[cur];
 #define GF2L_CNG(MD, FI) \
-    hipLaunchKernelGGL((cn_group_kernel<MD, FI>), dim3(grid), dim3(kGroupThreads), 0, s, cv, groups, gs, c2v[cur], b_in)
+    hipLaunchKernelGGL((cn_group_kernel<MD, FI>), dim3(grid), dim3(kGroupThreads), 0, s, cv, groups, sp, gs, c2v[cur], b_in)
 #define GF2L_CNG_FIRST(MD) \
     do { if (it == 1) GF2L_CNG(MD, true); else GF2L_CNG(MD, false); } while (0)
         if (max_dc <= 8)
@@ -464,10 +514,10 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
             GF2L_CNG_FIRST(32);
 #undef GF2L_CNG_FIRST
 #undef GF2L_CNG
-        hipLaunchKernelGGL(vn_group_kernel, dim3(grid), dim3(kGroupThreads), 0, s, cv, groups, gs, c2v[cur], bel[cur], llr[cur],
+        hipLaunchKernelGGL(vn_group_kernel, dim3(grid), dim3(kGroupThreads), 0, s, cv, groups, sp, gs, c2v[cur], bel[cur], llr[cur],
                            hb[in], hb[out], map[cur], (uint32_t)it, (int)last, d_msg, d_iters, d_conv, d_synd);
         GF2L_HIP(ctx, hipGetLastError());
-        if (it % batch != 0 || last) continue;
+        if ((it % batch != 0 && !(quick && it == 2)) || last) continue;
         GF2L_HIP(ctx, hipMemcpyAsync(ws.h_count, running, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         GF2L_HIP(ctx, hipStreamSynchronize(s));
         const uint32_t left = ws.h_count[0];
@@ -496,7 +546,7 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
 static int group_buffers(gf2l_ctx *ctx, const CsrView &cv, uint32_t groups) {
     // lists ([2][frames]): frame maps of both regions, sources of a packing
     const size_t slots = (size_t)groups * 64u, both = slots + (slots / 2 + 63u) / 64u * 64u;
-    return ensure_buffers(ctx, 2 * slots, both * cv.nnz, 0, both * cv.n, (size_t)groups * (2 * (size_t)cv.n + 2 + group_grid(ctx, cv, groups)), both * cv.n);
+    return ensure_buffers(ctx, 2 * slots, both * cv.nnz, 0, both * cv.n, (size_t)groups * (2 * (size_t)cv.n + 2 + group_grid_most(ctx)), both * cv.n);
 }
 
 // Decoder driver of the CSR path (same semantics as decode_device's plain
@@ -504,7 +554,7 @@ static int group_buffers(gf2l_ctx *ctx, const CsrView &cv, uint32_t groups) {
 int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
                uint64_t *d_msg, uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd) {
     const CsrView &cv = code->csr;
-    if (use_groups(cv) && ctx->tune.frame_kernel != 1) {
+    if (use_groups(cv, F) && ctx->tune.frame_kernel != 1) {
         const uint32_t pass = std::min(groups_per_pass(cv), (uint32_t)(((uint64_t)F + 63u) / 64u));
         if (group_buffers(ctx, cv, pass) == GF2L_OK) {
             const size_t kw = (cv.k + 63u) / 64u;
@@ -520,6 +570,7 @@ int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_
     }
     hipStream_t s = ctx->stream;
     const size_t nw = (cv.n + 63) / 64;
+    const uint32_t syn_threads = std::min(kSynThreads, std::max(1u, (cv.m + 63u) / 64u) * 64u);
     // the context's reusable workspace: c2v [F][nnz], beliefs [F][n], hard bits [F][nw]
     const int rc = ensure_buffers(ctx, F, (size_t)F * std::max<uint64_t>(cv.nnz, 1), 0, (size_t)F * cv.n,
                                   (size_t)F * nw, 0);
@@ -540,7 +591,7 @@ int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_
         hipLaunchKernelGGL(vn_csr_kernel, dim3(grid), dim3(256), 0, s, cv, list, counts + cur, c2v, bel,
                            d_llr, hb, counts + nxt);
         const uint32_t g_syn = std::min<uint32_t>(F, (uint32_t)ctx->num_cus * 8u);
-        hipLaunchKernelGGL(syn_csr_kernel, dim3(g_syn), dim3(kSynThreads), nw * sizeof(uint64_t), s, cv, list,
+        hipLaunchKernelGGL(syn_csr_kernel, dim3(g_syn), dim3(syn_threads), nw * sizeof(uint64_t), s, cv, list,
                            counts + cur, lists + (size_t)nxt * F, counts + nxt, hb, it, (int)(it == max_it),
                            d_msg, d_iters, d_conv, d_synd);
         GF2L_HIP(ctx, hipGetLastError());
