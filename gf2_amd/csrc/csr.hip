@@ -437,9 +437,11 @@ group_move_kernel(const uint32_t *__restrict__ src, const float *__restrict__ in
 // of n = 2,000: 280 -> 201 us, of n = 300,000: 3.59 -> 3.39 ms), whole rows instead
 // of gathered floats elsewhere (n = 9,000, 500 frames: 2.57 -> 0.89 ms against the
 // kernels above).  A single frame of up to 128 variables has nothing to win: 86
-// against 112 us for n = 7, 155 against 138 for n = 128.
+// against 112 us for n = 7, 155 against 138 for n = 128.  One or two frames of 2^16
+// variables and more gain little (n = 300,000: 2.09 -> 2.01 and 2.28 -> 2.01 ms;
+// error-free 256 and 332 us stay below 385) and would take the memory of 64.
 static bool use_groups(const CsrView &cv, uint32_t frames) {
-    if (frames == 1 && cv.n <= 128) return false;
+    if ((frames == 1 && cv.n <= 128) || (frames <= 2 && cv.n >= (1u << 16))) return false;
     return cv.nnz > 0 && cv.m > 0 && cv.nnz < (1u << 20) && cv.n < (1u << 20);
 }
 static uint32_t group_grid_most(const gf2l_ctx *ctx) { return 8u * ((uint32_t)ctx->num_cus / 2u); }
@@ -464,10 +466,15 @@ static GroupSplit group_split(const gf2l_ctx *ctx, const CsrView &cv, uint32_t g
     const uint32_t four = (rows + 4u * waves - 1u) / (4u * waves), one = (rows + waves - 1u) / waves;
     return {std::min(grid / 8u, std::min(one, std::max(four, grid / 8u / rounds))), groups_split(ctx, cv, groups) ? 1u : 0u};
 }
-// Groups per pass: the workspace of a pass stays below 4 GiB (at least eight groups).
-static uint32_t groups_per_pass(const CsrView &cv) {
-    const size_t per_group = ((size_t)cv.nnz + 2 * (size_t)cv.n) * 64 * sizeof(float) * 3 / 2;
-    return (uint32_t)std::max<size_t>(8, ((size_t)4 << 30) / per_group);
+// Floats of a row of 64 frames' arrays over `groups` groups: the groups themselves
+// and, for the packed ones, half as many (a single group is never packed).
+static size_t group_slots(uint32_t groups) { return 64 * ((size_t)groups + groups / 2); }
+// Groups per pass: the workspace of a pass stays below 4 GiB (the longest codes:
+// 1.2 GB a group), and groups fit a dimension of the grid.
+static uint32_t groups_per_pass(const gf2l_ctx *ctx, const CsrView &cv) {
+    const size_t per_group = ((size_t)cv.nnz + 2 * (size_t)cv.n) * 96 * sizeof(float) +
+                             (2 * (size_t)cv.n + 2 + group_grid_most(ctx)) * sizeof(uint64_t) + 128 * sizeof(uint32_t);
+    return (uint32_t)std::max<size_t>(1, std::min<size_t>(65535, ((size_t)4 << 30) / per_group));
 }
 
 static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_t F, uint32_t max_it,
@@ -483,7 +490,7 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
     uint64_t *hb[2] = {ws.hb, ws.hb + (size_t)groups * cv.n}, *active[2] = {hb[1] + (size_t)groups * cv.n, nullptr};
     active[1] = active[0] + groups;
     uint64_t *unsat = active[1] + groups;
-    uint32_t *map[2] = {ws.lists, ws.lists + slots}, *src = ws.lists + 2 * slots, *running = ws.counts;
+    uint32_t *map[2] = {ws.lists, ws.lists + slots}, *src = map[1] + (group_slots(groups) - slots), *running = ws.counts;
     uint32_t cur = 0;
     hipLaunchKernelGGL(group_init_kernel, dim3((groups * 64u + 255) / 256), dim3(256), 0, s, active[0], map[0], groups, F);
     hipLaunchKernelGGL(group_llr_kernel, dim3((cv.n + 63u) / 64u, groups), dim3(256), 0, s, d_llr, llr[0], F, cv.n);
@@ -545,8 +552,9 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
 
 static int group_buffers(gf2l_ctx *ctx, const CsrView &cv, uint32_t groups) {
     // lists ([2][frames]): frame maps of both regions, sources of a packing
-    const size_t slots = (size_t)groups * 64u, both = slots + (slots / 2 + 63u) / 64u * 64u;
-    return ensure_buffers(ctx, 2 * slots, both * cv.nnz, 0, both * cv.n, (size_t)groups * (2 * (size_t)cv.n + 2 + group_grid_most(ctx)), both * cv.n);
+    const size_t slots = (size_t)groups * 64u, both = group_slots(groups);
+    return ensure_buffers(ctx, slots, both * cv.nnz, 0, both * cv.n,
+                          (size_t)groups * (2 * (size_t)cv.n + 2 + group_grid_most(ctx)), both * cv.n);
 }
 
 // Decoder driver of the CSR path (same semantics as decode_device's plain
@@ -555,7 +563,7 @@ int decode_csr(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, uint32_
                uint64_t *d_msg, uint32_t *d_iters, uint8_t *d_conv, uint8_t *d_synd) {
     const CsrView &cv = code->csr;
     if (use_groups(cv, F) && ctx->tune.frame_kernel != 1) {
-        const uint32_t pass = std::min(groups_per_pass(cv), (uint32_t)(((uint64_t)F + 63u) / 64u));
+        const uint32_t pass = std::min(groups_per_pass(ctx, cv), (uint32_t)(((uint64_t)F + 63u) / 64u));
         if (group_buffers(ctx, cv, pass) == GF2L_OK) {
             const size_t kw = (cv.k + 63u) / 64u;
             for (uint64_t f0 = 0; f0 < F; f0 += 64ull * pass) {
