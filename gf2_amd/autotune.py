@@ -19,11 +19,15 @@ the context tunables of gf2l_set_tuning / gf2l_set_path:
   path         automatic (whole frame in LDS when it fits), compressed check
                state, or one stored message per edge (single-code decoder);
                a path that cannot run the code is skipped
+  frame_kernel whole-frame and team kernels where they are faster, or the
+               general kernels only; the knobs above change the general
+               kernels, so where the others run they measure alike
   lds_groups   thread groups per workgroup of the LDS path (one frame per
                workgroup; group g takes block-rows and block-columns g,
                g + groups, ...): the block-row tiling of small codes, which
                trades threads per frame (latency hiding) against passes per
                iteration and lanes left idle by z; 0 is the library's choice
+               (the small codes' whole-frame kernel where it applies)
 By default a code whose automatic path is the LDS path tunes lds_groups, any
 other code path, wg_per_cu and chunk.
 
@@ -32,7 +36,9 @@ Eb/N0 (the iteration profile of the operating point matters) once per
 candidate, checks that every candidate returns the same results, and keeps
 the fastest.  Results are cached per code-shape key in a JSON file
 ($GF2_AMD_TUNING, default ~/.cache/gf2_amd/tuning.json) so a later process
-applies them without measuring.
+applies them without measuring.  The key names the set of kernels that was
+measured: a choice among earlier kernels (a path or thread groups that were as
+fast as the automatic choice) would keep a call from the ones that came since.
 """
 from __future__ import annotations
 
@@ -54,11 +60,14 @@ CANDIDATES: Dict[str, List[int]] = {
     "graph_iters": [2, 4, 8],
     "chunk": [0, 4, 8, 16],
     "path": [_lib.PATH_AUTO, _lib.PATH_STATE, _lib.PATH_STREAM],
+    "frame_kernel": [0, 1],
     "lds_groups": [0, 2, 3, 4, 5, 8],
 }
 _TUNE_KEYS = {"wg_per_cu": _lib.TUNE_WG_PER_CU, "xcd_map": _lib.TUNE_XCD_MAP,
               "graph_iters": _lib.TUNE_GRAPH_ITERS, "chunk": _lib.TUNE_CHUNK,
-              "lds_groups": _lib.TUNE_LDS_GROUPS}
+              "lds_groups": _lib.TUNE_LDS_GROUPS, "frame_kernel": _lib.TUNE_FRAME_KERNEL}
+# Part of the cache key; changes when a kernel that the knobs choose among is added.
+KERNELS = "k2"
 
 
 def default_cache_path() -> str:
@@ -84,7 +93,7 @@ def batch_bucket(frames: int) -> int:
 
 
 def shape_key(codes: Sequence[LdpcCode], frames: int, kind: str) -> str:
-    return f"{kind}:" + "|".join(code_key(c) for c in codes) + f":F{batch_bucket(frames)}"
+    return f"{kind}:" + "|".join(code_key(c) for c in codes) + f":F{batch_bucket(frames)}:{KERNELS}"
 
 
 class TuningCache:
@@ -180,7 +189,7 @@ def tune_code(code: LdpcCode, frames: int, ebn0_db: float, max_it: int = 50, rep
 
 
 def tune_codeset(cs, code_ids: np.ndarray, d_llr: DeviceBuffer, max_it: int = 50, repeats: int = 2,
-                 knobs: Sequence[str] = ("wg_per_cu", "chunk", "graph_iters"),
+                 knobs: Sequence[str] = ("frame_kernel", "wg_per_cu", "chunk", "graph_iters"),
                  cache: Optional[TuningCache] = None) -> dict:
     """Tunes the mixed-code decoder of a code set on a resident batch (d_llr
     packed as gf2l_decode_mixed_device expects)."""
