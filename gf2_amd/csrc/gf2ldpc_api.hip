@@ -147,7 +147,7 @@ static bool use_team(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F, uin
     // two 2595 -> 2750 us; with a second turn 128 frames at r 1/2 2.72 -> 2.92 ms).
     if (code->flood.nd) {
         if (flood_bytes(cv, code->flood) <= 80 * 1024) return a.team >= 4;
-        return turns == 1 && a.team > 1 && full;
+        return turns == 1 && (a.team > 2 || (a.team == 2 && full));
     }
     // The other codes against the STATE kernels.  One workgroup a frame: at every
     // batch size (DVB-T2 normal r 5/6 1000 frames 14.2 -> 8.6 ms, N = 24000 with
