@@ -61,7 +61,9 @@ namespace {
 constexpr uint32_t kFloodGroups = 2;
 constexpr uint32_t kFloodThreads = 768;  // two groups of up to 384 lanes
 constexpr float kFloodLimit = 1e30f;
-// Information inputs per row of the instantiations.
+// Information inputs per row of the instantiations.  Each runs rows of its number
+// and of one less without guards (rows of a balanced code differ by one); a code
+// between two of them runs the larger one, padded.
 #define GF2L_FLOOD_DEGREES                                                                              \
     GF2L_FLOOD(4) GF2L_FLOOD(5) GF2L_FLOOD(6) GF2L_FLOOD(8) GF2L_FLOOD(9) GF2L_FLOOD(10) GF2L_FLOOD(11) \
     GF2L_FLOOD(13) GF2L_FLOOD(15) GF2L_FLOOD(17) GF2L_FLOOD(21) GF2L_FLOOD(25)
@@ -593,7 +595,7 @@ int build_flood_plan(gf2l_ctx *ctx, gf2l_code *c) {
         cv.nb * cv.zw > 0xffffu)
         return GF2L_OK;
     const uint32_t kb = cv.nb - cv.mb;
-    uint32_t most = 0;
+    uint32_t most = 0, inputs = 0;
     for (uint32_t br = 0; br < cv.mb; ++br) {
         const uint32_t e0 = c->h_row_ptr[br], d = c->h_row_ptr[br + 1] - e0, np = br > 0 ? 2u : 1u;
         if (d <= np) return GF2L_OK;
@@ -602,11 +604,17 @@ int build_flood_plan(gf2l_ctx *ctx, gf2l_code *c) {
             return GF2L_OK;
         if (c->h_row_edge[e0 + d - np - 1].x >= kb) return GF2L_OK;
         most = std::max(most, d - np);
+        inputs += d - np;
     }
     uint32_t nd = 0;
 #define GF2L_FLOOD(ND) nd = !nd && ND >= most ? ND : nd;
     GF2L_FLOOD_DEGREES
 #undef GF2L_FLOOD
+    // Rows are loaded padded to nd inputs.  Where two thirds of them are padding the
+    // other kernels are faster from 256 frames on (N = 64800, rows of 1 to 25 inputs,
+    // 4.0 on average: 256 frames 1154 -> 1560 us, 7.4 on average: 1368 -> 1397, at
+    // high Eb/N0 308 -> 399; rows of 4 to 17, 12 on average: 1511 -> 1026).
+    if (cv.mb * nd > 3u * inputs) return GF2L_OK;
     const size_t fixed = flood_fixed_bytes(cv, flood_lanes(cv.z)) + 256;
     if (!nd || fixed >= ctx->lds_limit) return GF2L_OK;
     const uint32_t X = (uint32_t)std::min<size_t>(kb, (ctx->lds_limit - fixed) / (cv.z * sizeof(float)));

@@ -82,3 +82,25 @@ def test_dvb_batches_of_several_turns(ctx, rate, counts, quiet):
             got = decode(ctx, code, llr[:count], 12, mode)
             same(got, decode(ctx, code, llr[:count], 12, GENERAL), (rate, count, quiet, mode))
             same([x[:4] for x in got], want, (rate, count, quiet, mode, "oracle"))
+
+
+# rows of 1 to 25 information inputs: mostly padding in the whole-frame kernel
+@pytest.mark.parametrize("mb,kb,z,counts", [(40, 60, 128, (1, 70, 300)), (60, 120, 360, (1, 86, 200))])
+def test_staircase_codes_of_uneven_rows(ctx, mb, kb, z, counts):
+    rng = np.random.default_rng(6)
+    base = np.full((mb, kb + mb), -1, dtype=np.int32)
+    for r in range(mb):
+        for c in rng.choice(kb, 25 if r % 10 == 3 else 1 + r % 4, replace=False):
+            base[r, c] = rng.integers(0, z)
+        base[r, kb + r] = 0
+        if r:
+            base[r, kb + r - 1] = 0
+    n = (kb + mb) * z
+    code, oc = LdpcCode(QuasiCyclicLdpc(base, z), ctx), orc.Code.from_qc(base, z)
+    llr = zero_codeword_llrs(rng, max(counts), n, rng.choice([0.3, 0.5, 0.9], max(counts)))
+    want = oc.decode_batch(llr[:8], 15, threads=8)
+    for count in counts:
+        print("[gpu-case] uneven rows", z, count, flush=True)
+        got = decode(ctx, code, llr[:count], 15, 0)
+        same(got, decode(ctx, code, llr[:count], 15, GENERAL), (z, count))
+        same([x[:8] for x in got], [x[:count] for x in want], (z, count, "oracle"))
