@@ -500,8 +500,9 @@ static int decode_csr_groups(gf2l_ctx *ctx, const gf2l_code *code, const float *
     // Few frames of a short code: launches are all there is, so those that one
     // iteration decodes are asked for at once (error-free: n = 2,000, 1 to 64 frames
     // 75 -> 36 us, n = 64, 4,096 frames 77 -> 39; in noise n = 2,000, 16 frames 200
-    // -> 180; with 500 frames, or n = 9,000, the question costs 2% to 8% in noise).
-    const bool quick = cv.n <= 6000 && (uint64_t)cv.n * groups < 16000;
+    // -> 180; with n = 6,000, 100 frames, or n = 9,000, the question costs 2% to 8%
+    // in noise).
+    const bool quick = cv.n <= 6000 && (uint64_t)cv.n * groups < 10000;
     // the pass after the last iteration takes its parities and retires the rest
     for (uint64_t it = 1; it <= (uint64_t)max_it + 1; ++it) {
         const uint32_t in = (it - 1) & 1u, out = it & 1u;
