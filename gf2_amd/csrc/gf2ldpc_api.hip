@@ -156,12 +156,13 @@ static bool use_team(const gf2l_ctx *ctx, const gf2l_code *code, uint32_t F, uin
     if (a.team == 1 || turns == 1) return true;
     // Several turns of larger teams: where the STATE kernels are slow, in full
     // turns.  They hold back with many messages a variable (DVB-T2 normal r 2/3,
-    // columns of 13: 1000 frames 22.7 -> 15.0 ms, 500 11.2 -> 8.0, but 150 frames,
+    // columns of 13: 1000 frames 22.7 -> 14.5 ms, 500 11.2 -> 7.6, but 150 frames,
     // a second turn of 22, 3.82 -> 3.86 ms) and with short block-rows (N = 64768
     // with z = 128, 256 frames 3.94 -> 3.03 ms, z = 64 6.13 -> 3.18, and there also
     // with short turns: 90 frames 2.66 -> 1.67 ms).  Otherwise they catch up with
     // the number of frames (DVB-T2 normal r 1/2, columns of 8: 170 frames 4.36 ->
-    // 3.44 ms, 500 10.2 -> 9.1, 1000 at 0.6 dB more 9.4 -> 10.0; N = 64800 with
+    // 3.14 ms, 500 10.2 -> 8.3, 1000 at 1.5 dB more, when the teams started again,
+    // 5.95 -> 6.90; N = 64800 with
     // z = 360 and no staircase: 1024 frames 10.4 -> 11.1 ms).
     if (cv.z <= 64) return true;
     return full && (cv.max_dv > 8 || cv.z <= 128 || (cv.dvb_q && turns <= 6));
@@ -249,6 +250,7 @@ static int decode_team(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr,
     a.llr_own = ws.llr_perm;
     a.msg = ws.c2v;
     a.bel = ws.belief;
+    a.state = list && a.team > 1 && team_resumes(cv) ? reinterpret_cast<const uint3 *>(ws.state) : nullptr;
     a.sync = ws.hb;
     a.gave_up = ws.counts;
     a.queue = ws.counts + 1;
@@ -352,8 +354,8 @@ int decode_device(gf2l_ctx *ctx, const gf2l_code *code, const float *d_llr, size
                 // DVB codes whose teams take several frames each: the first
                 // iteration by the state kernels, which are faster at it (202
                 // error-free frames of DVB-T2 normal r 3/5: 265 us, 345 by teams;
-                // in noise the teams alone would take 3% to 16% less), then teams
-                // for the frames still running.
+                // in noise the teams alone take up to 9% less, at r 4/5 20%, at r
+                // 1/2 4% more), then teams for the frames still running.
                 int rc1 = ensure_workspace(ctx, cv, path, F);
                 if (rc1 == GF2L_OK) rc1 = team_buffers(ctx, cv, team, F);
                 if (rc1 == GF2L_OK)

@@ -200,7 +200,8 @@ struct TeamArgs {
     size_t llr_words;        // otherwise floats of llr_own
     float *llr_own;          // per workgroup, by owning thread
     float *msg;              // per team [nbe][zp] check messages
-    float *bel;              // per team [nb][zp] beliefs
+    float *bel;              // per team [nb][zp] beliefs (with state: per frame)
+    const uint3 *state;      // per frame [mb][zp] check states after iteration 1, to go on from (null: from the LLRs)
     uint64_t *sync;          // per team, kTeamSyncStride apart: meeting counter (zeroed before the launch)
     uint32_t *queue;         // frames taken past the first of each team (zeroed before the launch)
     uint32_t *gave_up;       // set when a wait ended without the team (zeroed before the launch)
@@ -424,6 +425,7 @@ hipError_t launch_flood_mix(const FloodMixArgs &a, size_t lds, uint32_t block, u
 // suit the code or the batch) and the launcher.
 bool team_shape(const CodeView &cv, uint32_t frames, uint32_t max_it, int num_cus, size_t lds_limit, TeamArgs &a);
 hipError_t launch_team(const TeamArgs &a, hipStream_t s);
+bool team_resumes(const CodeView &cv);  // whether its teams go on from the state kernels' states (TeamArgs::state)
 
 // Whole-frame kernel of small codes on the LDS path (small.hip): its workgroup
 // for a code (0: the code does not suit it) and the launcher.  ctr: two words,

@@ -65,14 +65,14 @@ def test_codes_without_staircase(ctx, mb, nb, z, counts):
         same([x[:12] for x in got], [x[:count] for x in want], (z, count, "oracle"))
 
 
-# teams of three (85 at a time) and two (128 at a time)
-@pytest.mark.parametrize("rate,counts", [(0, (86, 128, 520)), (2, (129, 200))])
+# teams of three (85 at a time) and two (128 at a time); checks up to 8, 16 and 27
+@pytest.mark.parametrize("rate,counts", [(0, (86, 128, 520)), (2, (129, 200)), (4, (250,))])
 @pytest.mark.parametrize("quiet", [0.0, 0.1, 0.4])  # share of frames that one iteration decodes
 def test_dvb_batches_of_several_turns(ctx, rate, counts, quiet):
     code, s = LdpcCode.dvb_t2_normal(CodeRate(rate), ctx), codes.dvb_t2(1, rate)
     oc = orc.Code(s.m, s.n, orc.dvb_edges(s.table, s.n, s.k, s.q))
     rng = np.random.default_rng(5)
-    noisy = zero_codeword_llrs(rng, 40, s.n, 0.75 if rate == 0 else 0.6)
+    noisy = zero_codeword_llrs(rng, 40, s.n, {0: 0.75, 2: 0.6, 4: 0.53}[rate])
     llr = noisy[rng.integers(0, 40, max(counts))]
     llr[rng.random(max(counts)) < quiet] = 10.0
     want = oc.decode_batch(llr[:4], 12, threads=8)
