@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(512) lnms_fwd_kernel(LayeredArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Staircase kernel (decoding only).  For a QC-IRA code whose parity part is a
+// Staircase kernel (decoding, and the training forward: TAPE).  For a QC-IRA code whose parity part is a
 // block staircase of unshifted circulants (block-row r has the parity
 // block-columns kb+r-1 and kb+r as its last two edges, shift 0), check i of
 // every block-row touches parity bit i of its parity columns: those beliefs

@@ -15,9 +15,11 @@
 // frames: 1440 -> 480 us, bound by the exchange (3.4 MB a frame and iteration at
 // 5 TB/s).
 //
-// Exchange: a team's workgroups sit on different XCDs, whose L2s are not
-// coherent within a kernel, so messages and beliefs are stored and loaded at
-// agent scope, and a workgroup reports to the counter when its stores are done.
+// Exchange: a team's workgroups may sit on different XCDs (workgroup b on XCD
+// b % 8: they all share one only where the number of teams is a multiple of 8),
+// whose L2s are not coherent within a kernel, so messages and beliefs are stored
+// and loaded at agent scope, and a workgroup reports to the counter when its
+// stores are done.
 // Plain loads with an acquire fence at each meeting were slower (24 frames: 1.93
 // ms, each fence drops the caches of the whole XCD).
 //
