@@ -201,7 +201,6 @@ struct TeamArgs {
     float *llr_own;          // per workgroup, by owning thread
     float *msg;              // per team [nbe][zp] check messages
     float *bel;              // per team [nb][zp] beliefs (with state: per frame)
-    const uint3 *state;      // per frame [mb][zp] check states after iteration 1, to go on from (null: from the LLRs)
     uint64_t *sync;          // per team, kTeamSyncStride apart: meeting counter (zeroed before the launch)
     uint32_t *queue;         // frames taken past the first of each team (zeroed before the launch)
     uint32_t *gave_up;       // set when a wait ended without the team (zeroed before the launch)
@@ -209,6 +208,7 @@ struct TeamArgs {
     uint64_t *msg_out;
     uint32_t *iters;
     uint8_t *conv, *synd;
+    const uint3 *state;      // per frame [mb][zp] check states after iteration 1, to go on from (null: from the LLRs)
 };
 constexpr uint32_t kTeamSyncStride = 16;
 
