@@ -75,13 +75,16 @@ def test_dvb_batches_of_several_turns(ctx, rate, counts, quiet):
     noisy = zero_codeword_llrs(rng, 40, s.n, {0: 0.75, 2: 0.6, 4: 0.53}[rate])
     llr = noisy[rng.integers(0, 40, max(counts))]
     llr[rng.random(max(counts)) < quiet] = 10.0
-    want = oc.decode_batch(llr[:4], 12, threads=8)
-    for count in counts:
-        for mode in (0, TEAM_NO_WAIT):  # with and without teams that leave after the first iteration
-            print("[gpu-case] team turns", rate, count, quiet, mode, flush=True)
-            got = decode(ctx, code, llr[:count], 12, mode)
-            same(got, decode(ctx, code, llr[:count], 12, GENERAL), (rate, count, quiet, mode))
-            same([x[:4] for x in got], want, (rate, count, quiet, mode, "oracle"))
+    llr[rng.random(llr.shape) < 0.001] = -0.0
+    llr[1, :3], llr[2, 7] = [np.inf, -np.inf, 1e38], np.nan
+    for max_it in (2, 12):
+        want = oc.decode_batch(llr[:4], max_it, threads=8)
+        for count in counts:
+            for mode in (0, TEAM_NO_WAIT):  # with and without teams that leave after the first iteration
+                print("[gpu-case] team turns", rate, count, quiet, max_it, mode, flush=True)
+                got = decode(ctx, code, llr[:count], max_it, mode)
+                same(got, decode(ctx, code, llr[:count], max_it, GENERAL), (rate, count, quiet, max_it, mode))
+                same([x[:4] for x in got], want, (rate, count, quiet, max_it, mode, "oracle"))
 
 
 # rows of 1 to 25 information inputs: mostly padding in the whole-frame kernel
